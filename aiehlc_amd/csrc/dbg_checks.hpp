@@ -71,7 +71,7 @@ constexpr uint32_t file_id(const char* s) {
 }
 constexpr const char* kFiles[] = {"gemm_i8_kernels.hpp", "gemm_i8.hip",       "gemm_bf16.hip",   "conv2d_i8.hip",
                                   "conv2d_i8_rows.hpp",  "gfx950_ops.hpp",    "ref_kernels.hip", "miaie_runtime.hip",
-                                  "dbg_checks.hpp",      "noalloc.hip"};
+                                  "dbg_checks.hpp",      "noalloc.hip",       "flex_tile.hpp"};
 
 // One translation unit's table and record, as the runtime drives them.
 struct Unit {

@@ -23,10 +23,11 @@
 //                   at a higher clock than the 32x32 form under the power
 //                   limit; gemm_i8_pipe16_mixed puts 256x256 and 256x128
 //                   tiles in one launch.
-//   gemm_i8_tile64p 64x64x64 tile for K % 16 == 0 and 16-byte aligned rows:
-//                   clamped vector loads, next k-tile prefetched into
-//                   registers.
-//   gemm_i8_tile64  64x64x64 tile, bounds-checked, any shape / stride.
+//   gemm_i8_flex    register-staged 16x128, 64x64 and 128x128 tiles
+//                   (flex_tile.hpp) for every other shape, stride and
+//                   alignment with rows of at least 16 bytes; K split over
+//                   workgroups where tiles are few.
+//   gemm_i8_tile64  64x64x64 tile, bounds-checked, for rows below 16 bytes.
 // The requantize epilogue (round, shift, saturate, optional ReLU) is fused
 // into all of them.
 //
@@ -35,6 +36,7 @@
 // one dword of int8 output or one 16-byte int32 vector per 4 values.
 #include <type_traits>
 
+#include "flex_tile.hpp"
 #include "gemm_i8_kernels.hpp"
 #include "gfx950_ops.hpp"
 #include "miaie_internal.hpp"
@@ -45,9 +47,10 @@ namespace dev = miaie::dev;
 using namespace miaie::gemm;
 using miaie::kernel_t;
 using miaie::launch;
+namespace flex = miaie::flex;
 
 // ------------------------------------------------------------ 64x64 tile
-// Bounds-checked fallback for shapes and strides the 256 kernel does not take.
+// Bounds-checked fallback for rows of fewer than 16 bytes.
 template <bool B_NT>
 __global__ __launch_bounds__(256) void gemm_i8_tile64(const int8_t* __restrict__ A,
                                                       const int8_t* __restrict__ B,
@@ -133,80 +136,67 @@ __global__ __launch_bounds__(256) void gemm_i8_tile64(const int8_t* __restrict__
   }
 }
 
-// The 64x64 kernel for K % 16 == 0 and 16-byte aligned operands (a ragged M,
-// N or K): every load is a full vector from a clamped, always valid address,
-// zeroed when written to LDS if outside the matrix, and the next k-tile's
-// loads are issued before this k-tile's LDS reads and MFMAs, so their
-// latency overlaps the MFMAs (a load under a condition, or zeroed in place,
-// would be waited for on the spot).
-template <bool B_NT>
-__global__ __launch_bounds__(256) void gemm_i8_tile64p(const int8_t* __restrict__ A,
-                                                       const int8_t* __restrict__ B,
-                                                       int8_t* __restrict__ Y, int32_t* __restrict__ C,
-                                                       int M, int N, int K, int lda, int ldb, int ldy,
-                                                       int ldc, int shift, int relu) {
-  __shared__ __attribute__((aligned(16))) int8_t as[64 * 64];
-  __shared__ __attribute__((aligned(16))) int8_t bs[64 * 64];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int fr = lane & 31, fh = lane >> 5;
+// Register-staged tiles (flex_tile.hpp): any size, stride and alignment with
+// rows of at least 16 bytes.  grid.x: output tiles, grid.y: the `splits`
+// workgroups that divide a tile's K.  Bound by the latency of the stages'
+// loads, and for few rows by reading B: 1000 x 2050 x 1000 NT (rows of 1000
+// bytes) took 61.1 us in the byte-wise 64x64 kernel and takes 8.8; the MLP
+// over 16 rows (4096 -> 11008 -> 4096, 90 MB of weights) 204.7 us in a
+// vectorised 64x64 kernel without a split and 29.2 (27.3 with K split 8
+// ways, 72 unsplit, on one box).
+template <class G, bool B_NT>
+__global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void gemm_i8_flex(const int8_t* __restrict__ A, const int8_t* __restrict__ B,
+                                                       int8_t* __restrict__ Y, int32_t* __restrict__ C, int M, int N,
+                                                       int K, int lda, int ldb, int ldy, int ldc, int shift, int relu,
+                                                       int8_t* __restrict__ work, uint32_t* __restrict__ counters) {
+  __shared__ __attribute__((aligned(1024))) int8_t lds[G::LDS];
+  __shared__ int flag;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / G::WAVES_N, wn = wave % G::WAVES_N;
+  int tm, tn;
+  dev::tile_coords<4>(blockIdx.x, (M + G::BM - 1) / G::BM, (N + G::BN - 1) / G::BN, tm, tn);
+  const int m0 = tm * G::BM, n0 = tn * G::BN;
+  const int stages = (K + G::KB - 1) / G::KB, splits = gridDim.y, split = blockIdx.y;
+  const int s0 = (int)((long long)stages * split / splits), s1 = (int)((long long)stages * (split + 1) / splits);
 
-  // A (and NT B): thread -> row tid/4, 16-byte chunk tid%4.  K % 16 == 0, so
-  // a chunk lies wholly inside or wholly past K; one past K loads the last
-  // chunk of its row instead and is zeroed like a row outside the matrix.
-  const int row = tid >> 2, ch = tid & 3;
-  const bool a_in = m0 + row < M;
-  const int8_t* const a_p = A + (size_t)min(m0 + row, M - 1) * lda;
-  // NT B: row n0 + row; NN B: column n0 + tid%64, k-chunk tid/64 (16 byte loads down the column)
-  const int bcol = tid & 63, bch = tid >> 6;
-  const bool b_in = B_NT ? n0 + row < N : n0 + bcol < N;
-  const int8_t* const b_p = B_NT ? B + (size_t)min(n0 + row, N - 1) * ldb : B + min(n0 + bcol, N - 1);
-  const int bk = B_NT ? ch : bch;  // this thread's k-chunk of B
-
-  auto load = [&](int k0, v4i& va, v4i& vb) {
-    va = MIAIE_LD(reinterpret_cast<const v4i*>(a_p + min(k0 + 16 * ch, K - 16)));
-    if constexpr (B_NT) {
-      vb = MIAIE_LD(reinterpret_cast<const v4i*>(b_p + min(k0 + 16 * ch, K - 16)));
-    } else {
-      const int8_t* const p = b_p + (size_t)min(k0 + 16 * bch, K - 16) * ldb;
-      int8_t tmp[16];
+  v4i acc[G::NI][G::NJ];
 #pragma unroll
-      for (int t = 0; t < 16; ++t) tmp[t] = MIAIE_LD(p + (size_t)t * ldb);
-      __builtin_memcpy(&vb, tmp, 16);
-    }
-  };
-
-  v16i acc = v16i{0};
-  v4i va, vb;
-  load(0, va, vb);
-  for (int k0 = 0; k0 < K; k0 += 64) {
-    *reinterpret_cast<v4i*>(as + lds_off(row, ch)) = a_in && k0 + 16 * ch < K ? va : v4i{0};
-    if constexpr (B_NT)
-      *reinterpret_cast<v4i*>(bs + lds_off(row, ch)) = b_in && k0 + 16 * bk < K ? vb : v4i{0};
-    else
-      *reinterpret_cast<v4i*>(bs + lds_off(bcol, bch)) = b_in && k0 + 16 * bk < K ? vb : v4i{0};
-    __syncthreads();
-    if (k0 + 64 < K) load(k0 + 64, va, vb);
+  for (int i = 0; i < G::NI; ++i)
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      const v4i af = *reinterpret_cast<const v4i*>(as + lds_off(wm * 32 + fr, 2 * ks + fh));
-      const v4i bf = *reinterpret_cast<const v4i*>(bs + lds_off(wn * 32 + fr, 2 * ks + fh));
-      acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf, af, acc, 0, 0, 0);
-    }
-    __syncthreads();
+    for (int j = 0; j < G::NJ; ++j) acc[i][j] = v4i{0};
+  flex::RowsLoader<G, G::NA> la(A, m0, M, lda, K, tid);
+  if constexpr (B_NT) {
+    flex::RowsLoader<G, G::NB> lb(B, n0, N, ldb, K, tid);
+    flex::tile_loop<int8_t, G, false>(lds, la, lb, s0, s1, lane, wm, wn, acc);
+  } else {
+    flex::ColsLoader<int8_t, G, false> lb(B, n0, N, ldb, K, tid);
+    flex::tile_loop<int8_t, G, true>(lds, la, lb, s0, s1, lane, wm, wn, acc);
   }
+  if (splits > 1 &&
+      !flex::split_sum<int8_t, G>(acc, blockIdx.x, split, splits, work, counters, &flag, tid))
+    return;
 
-  const int m = m0 + wm * 32 + fr;
-  if (m >= M) return;
+  const int fr = lane & 15, fg = lane >> 4, lo = relu ? 0 : -128;
+  const Requant rq{shift, shift ? 1 << (shift - 1) : 0, lo, 127};
 #pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    const int n = n0 + wn * 32 + 8 * (e >> 2) + 4 * fh + (e & 3);
-    if (n < N) {
-      if (C) MIAIE_ST(C + (size_t)m * ldc + n, acc[e]);
-      if (Y) MIAIE_ST(Y + (size_t)m * ldy + n, (int8_t)requant1(acc[e], shift, relu));
+  for (int i = 0; i < G::NI; ++i)
+#pragma unroll
+    for (int j = 0; j < G::NJ; ++j) {
+      const int ml = wm * G::WM + 16 * i + fr, nl = wn * G::WN + 16 * j + 4 * fg;
+      const v4i& a = acc[i][j];
+      if (C) flex::store4(C, ldc, m0 + ml, n0 + nl, M, N, a);
+      uint32_t y = 0;
+      if (K < (1 << 16)) {  // |acc| + 2^30 < 2^31
+        y = rq.pack4(a[0], a[1], a[2], a[3]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y |= (uint32_t)(requant1(a[e], shift, relu) & 0xFF) << (8 * e);
+      }
+      *reinterpret_cast<uint32_t*>(lds + ml * G::YP + nl) = y;
     }
-  }
+  if (!Y) return;
+  __syncthreads();
+  flex::store_y<G>(lds, Y, ldy, m0, n0, M, N, tid);
 }
 
 // keep_y: the caller reads Y right after (the MLP's H): ordinary stores that
@@ -425,6 +415,12 @@ static bool pipe_operands_ok(const int8_t* A, const int8_t* B, const int8_t* Y, 
          (!C || (aligned(C, 16) && ldc % 4 == 0));
 }
 
+// The register-staged kernel's conditions: rows of at least 16 bytes, and
+// 32-bit offsets within a tile.
+static bool flex_operands_ok(int N, int K, int lda, int ldb, int b_nt) {
+  return K >= 16 && (b_nt || N >= 16) && lda < (1 << 25) && ldb < (1 << 25);
+}
+
 int plan_gemm_i8(miaie_ctx* ctx, int M, int N, int K, int dense_ok, miaie_gemm_plan* plan) {
   const PipePlan p = dense_ok ? plan_pipe(M, N, K, ctx->cus) : PipePlan{};
   *plan = miaie_gemm_plan{};
@@ -439,6 +435,12 @@ int plan_gemm_i8(miaie_ctx* ctx, int M, int N, int K, int dense_ok, miaie_gemm_p
     plan->tile_m = p.bm;
     plan->tile_n = p.bn;
     plan->workgroups = ((M + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn);
+  } else if (flex_operands_ok(N, K, K, N, false)) {
+    const flex::Plan f = flex::plan(M, N, K, 1.0, ctx->cus, true, ctx->work_bytes);
+    plan->kernel = MIAIE_KERNEL_TILE64;
+    plan->tile_m = f.bm;
+    plan->tile_n = f.bn;
+    plan->workgroups = (int)(f.tiles * f.splits);
   } else {
     plan->kernel = MIAIE_KERNEL_TILE64;
     plan->tile_m = 64;
@@ -451,21 +453,20 @@ int plan_gemm_i8(miaie_ctx* ctx, int M, int N, int K, int dense_ok, miaie_gemm_p
 // Chooses the kernel.  Y and/or C may be NULL (not both).
 int launch_gemm_i8(miaie_ctx* ctx, const int8_t* A, const int8_t* B, int8_t* Y, int32_t* C, int M,
                    int N, int K, int lda, int ldb, int ldy, int ldc, int b_nt, int shift, int relu, bool keep_y) {
-  miaie_gemm_plan plan;
-  const bool dense_ok = pipe_operands_ok(A, B, Y, C, K, lda, ldb, ldy, ldc);
-  plan_gemm_i8(ctx, M, N, K, dense_ok, &plan);
-  if (plan.kernel == MIAIE_KERNEL_PIPE_MIXED) {
-    const int nw = plan_pipe(M, N, K, ctx->cus).nw;
-    const int dev = ctx->device;
+  const PipePlan plan =
+      pipe_operands_ok(A, B, Y, C, K, lda, ldb, ldy, ldc) ? plan_pipe(M, N, K, ctx->cus) : PipePlan{};
+  const int dev = ctx->device;
+  if (plan.bm && plan.nw) {
+    const int nw = plan.nw;
     const hipError_t e =
         b_nt ? launch_pipe_mixed<true>(dev, ctx->stream, A, B, Y, C, M, N, K, lda, ldb, ldy, ldc, shift, relu, nw, keep_y)
              : launch_pipe_mixed<false>(dev, ctx->stream, A, B, Y, C, M, N, K, lda, ldb, ldy, ldc, shift, relu, nw,
                                         keep_y);
     return check_launch(ctx, e, "gemm_i8_pipe16_mixed");
   }
-  if (plan.kernel == MIAIE_KERNEL_PIPE) {
+  if (plan.bm) {
     hipStream_t st = ctx->stream;
-    const int dev = ctx->device, bm = plan.tile_m, bn = plan.tile_n;
+    const int bm = plan.bm, bn = plan.bn;
     hipError_t e;
     if (bm == 256 && bn == 256)
       e = b_nt ? launch_pipe<256, 256, true>(dev, st, A, B, Y, C, M, N, K, lda, ldb, ldy, ldc, shift, relu, keep_y)
@@ -480,16 +481,20 @@ int launch_gemm_i8(miaie_ctx* ctx, const int8_t* A, const int8_t* B, int8_t* Y, 
   }
   dim3 grid((N + 63) / 64, (M + 63) / 64), block(256);
   if (grid.y > 65535) return fail(ctx, MIAIE_EINVAL, "gemm_i8: M too large for the 64x64 fallback");
-  // vector loads need K % 16 == 0 and 16-byte aligned A (and NT B) rows
-  const bool vec = K % 16 == 0 && aligned(A, 16) && lda % 16 == 0 && (!b_nt || (aligned(B, 16) && ldb % 16 == 0));
-  const int dev = ctx->device;
-  if (vec) {
-    const hipError_t e =
-        b_nt ? launch<gemm_i8_tile64p<true>>(dev, grid, block, 0, ctx->stream, A, B, Y, C, M, N, K, lda, ldb, ldy,
-                                             ldc, shift, relu)
-             : launch<gemm_i8_tile64p<false>>(dev, grid, block, 0, ctx->stream, A, B, Y, C, M, N, K, lda, ldb, ldy,
-                                              ldc, shift, relu);
-    return check_launch(ctx, e, "gemm_i8_tile64p");
+  if (flex_operands_ok(N, K, lda, ldb, b_nt)) {
+    flex::Plan f = flex::plan(M, N, K, 1.0, ctx->cus, true, ctx->work_bytes);
+    if (f.splits > 1 && !may_split(ctx)) f = flex::plan(M, N, K, 1.0, ctx->cus, false, 0);
+    hipError_t e = hipSuccess;
+    flex::with_geom(f, [&](auto g) {
+      using G = typename decltype(g)::type;
+      const dim3 fg((unsigned)f.tiles, (unsigned)f.splits);
+      int8_t* const work = static_cast<int8_t*>(ctx->work);
+      e = b_nt ? launch<gemm_i8_flex<G, true>>(dev, fg, block, 0, ctx->stream, A, B, Y, C, M, N, K, lda, ldb, ldy, ldc,
+                                               shift, relu, work, ctx->counters)
+               : launch<gemm_i8_flex<G, false>>(dev, fg, block, 0, ctx->stream, A, B, Y, C, M, N, K, lda, ldb, ldy, ldc,
+                                                shift, relu, work, ctx->counters);
+    });
+    return check_launch(ctx, e, "gemm_i8_flex");
   }
   const hipError_t e =
       b_nt ? launch<gemm_i8_tile64<true>>(dev, grid, block, 0, ctx->stream, A, B, Y, C, M, N, K, lda, ldb, ldy, ldc,

@@ -23,14 +23,17 @@ struct miaie_ctx {
   bool recording = false;     // between miaie_graph_begin and miaie_graph_end
   void* scratch = nullptr;    // device address of this device's file-scope scratch array (noalloc.hip)
   // Device workspace owned by this context, allocated once at init so that
-  // no entry point allocates: the conv's split-K partial sums.  Work queued
-  // on the context's one stream uses it in stream order.
+  // no entry point allocates: split-K partial sums, and the arrival counters
+  // of the tiles whose K is split (flex::split_sum; every launch leaves them
+  // at 0).  Work queued on the context's one stream uses it in stream order.
   void* work = nullptr;
   size_t work_bytes = 0;
+  uint32_t* counters = nullptr;  // MIAIE_CTX_COUNTERS of them, behind the work_bytes
   char err[512] = {0};
 };
 
 constexpr size_t MIAIE_CTX_WORK_BYTES = (size_t)16 << 20;
+constexpr int MIAIE_CTX_COUNTERS = 4096;
 
 namespace miaie {
 
@@ -94,6 +97,11 @@ struct kernel_t {
   static constexpr auto value = K;
 };
 
+template <class T>
+struct type_t {
+  using type = T;
+};
+
 // Every entry point starts with this: non-null context, its device current.
 int enter(miaie_ctx* ctx);
 
@@ -119,6 +127,12 @@ int scratch_setup(miaie_ctx* ctx);
 // Validated chained MLP over a caller-chosen H (capi.hip).
 int mlp_i8_checked(miaie_ctx* ctx, const char* fn, const int8_t* X, const int8_t* W1, const int8_t* W2, int8_t* H,
                    int8_t* Y, int M, int K, int F, int Nout, int s1, int s2);
+
+// Whether a launch may keep split-K partial sums in the context's workspace:
+// not while the caller itself captures the context's stream (its graph could
+// be replayed beside other work of the context; chains recorded with
+// miaie_graph_begin replay on the context's own stream only).
+bool may_split(miaie_ctx* ctx);
 
 // ---- kernel launchers implemented in the kernel translation units ----
 // keep_y: Y is read by the next kernel (ordinary stores instead of

@@ -60,6 +60,12 @@ int refuse_while_recording(miaie_ctx* ctx, const char* what) {
   return MIAIE_OK;
 }
 
+bool may_split(miaie_ctx* ctx) {
+  if (ctx->recording || !ctx->stream) return true;  // (the null stream cannot be captured)
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(ctx->stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+}
+
 // ---------------------------------------------------------------- device bounds checks
 // The buffer table of the debug build (dbg_checks.hpp): one process-wide map
 // of [lo, hi) ranges, uploaded into every translation unit's copy of the
@@ -256,17 +262,24 @@ extern "C" int miaie_init_on_stream(miaie_ctx** out, int device, void* stream) {
     delete ctx;
     return rc;
   }
-  e = hipMalloc(&ctx->work, MIAIE_CTX_WORK_BYTES);
+  constexpr size_t kCounterBytes = MIAIE_CTX_COUNTERS * sizeof(uint32_t);
+  e = hipMalloc(&ctx->work, MIAIE_CTX_WORK_BYTES + kCounterBytes);
+  if (e == hipSuccess) {
+    ctx->work_bytes = MIAIE_CTX_WORK_BYTES;
+    ctx->counters = reinterpret_cast<uint32_t*>(static_cast<int8_t*>(ctx->work) + MIAIE_CTX_WORK_BYTES);
+    e = hipMemset(ctx->counters, 0, kCounterBytes);
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);  // done before any stream uses them
+  }
   if (e != hipSuccess) {
     int rc = hip_fail(nullptr, e, "hipMalloc (context workspace)");
+    if (ctx->work) (void)hipFree(ctx->work);
     (void)hipEventDestroy(ctx->done);
     delete ctx;
     return rc;
   }
-  ctx->work_bytes = MIAIE_CTX_WORK_BYTES;
   // (debug build) the workspace and the scratch array are buffers the
   // kernels may touch
-  int rc = dbg_add(ctx, ctx->work, ctx->work_bytes);
+  int rc = dbg_add(ctx, ctx->work, ctx->work_bytes + kCounterBytes);
   if (rc == MIAIE_OK) rc = dbg_add(ctx, ctx->scratch, MIAIE_MLP_NOALLOC_MAX_H);
   if (rc != MIAIE_OK) {
     fail(nullptr, rc, "%s", ctx->err);

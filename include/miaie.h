@@ -52,8 +52,9 @@ typedef struct miaie_ctx miaie_ctx;
 /* Replaces XAie_SetupConfig + XAie_CfgInitialize + XAie_PartitionInitialize
  * (example/perf/aieml_perf.cc:265-313).  Binds `device` and creates a
  * stream owned by the context.  It also allocates the context's 16 MiB
- * device workspace (split-K partial sums of deep convolutions), released by
- * miaie_finish, so that no compute entry point allocates. */
+ * device workspace (partial sums of products whose K is split over
+ * workgroups), released by miaie_finish, so that no compute entry point
+ * allocates. */
 MIAIE_API int miaie_init(miaie_ctx** ctx, int device);
 
 /* As miaie_init, but launches go to the caller's hipStream_t `stream`
@@ -121,7 +122,8 @@ MIAIE_API int miaie_debug_unregister(miaie_ctx* ctx, const void* dev_ptr);
 
 /* ---- GEMM planning ------------------------------------------------------ */
 
-#define MIAIE_KERNEL_TILE64 0     /* bounds-checked 64x64 kernel, any shape and stride */
+#define MIAIE_KERNEL_TILE64 0     /* register-staged kernel, any shape and stride: tiles of 16x128, 64x64 or
+                                     128x128, K split over workgroups where tiles are few */
 #define MIAIE_KERNEL_PIPE 1       /* pipelined tile_m x tile_n kernel, 4-stage LDS DMA pipeline; M >= tile_m,
                                      N >= tile_n, and N % 16 == 0 where tile_n does not divide N (the
                                      last tile row/column overlaps the one before it) */
@@ -133,7 +135,8 @@ MIAIE_API int miaie_debug_unregister(miaie_ctx* ctx, const void* dev_ptr);
  * decomposition and tile choice that stand in for the reference's tiling
  * prototype, src/mlir/mlirfront/tilinglinalg/tilinglinalg.cpp:38-146).
  * miaie_gemm_i8_i32 runs the same plan, except that for K >= 2^16, where the
- * requantizing entry takes the 64x64 kernel, it keeps the pipelined one. */
+ * requantizing entry takes the register-staged kernel, it keeps the pipelined
+ * one. */
 typedef struct {
   int kernel;         /* MIAIE_KERNEL_* */
   int tile_m, tile_n; /* workgroup output tile */
@@ -184,8 +187,9 @@ MIAIE_API int miaie_plan_conv2d_i8(int N, int H, int W, int Cin, int Cout, int R
  * (MIAIE_EUNSUPPORTED).  miaie_graph_launch queues one replay on the
  * context's stream (asynchronous, like any launch).  A graph replays only on
  * the context that recorded it (another context gets MIAIE_EINVAL), before
- * that context's miaie_finish: a recorded convolution may use the context's
- * workspace. */
+ * that context's miaie_finish: a recorded product or convolution may use the
+ * context's workspace.  (While the caller captures the context's stream with
+ * HIP itself, GEMMs are not split over K and so leave the workspace alone.) */
 typedef struct miaie_graph miaie_graph;
 MIAIE_API int miaie_graph_begin(miaie_ctx* ctx);
 MIAIE_API int miaie_graph_end(miaie_ctx* ctx, miaie_graph** graph);

@@ -1,0 +1,118 @@
+"""The register-staged tiles (csrc/flex_tile.hpp): int8 GEMM for every shape,
+stride and alignment the pipelined kernels do not take, with K split over
+workgroups where tiles are few.  Sizes at the edges of the tiles (16 x 128,
+64 x 64, 128 x 128), of the 16-byte chunks and of the 256-byte stages; each call
+is repeated, since a split leaves its arrival counters for the next launch."""
+import numpy as np
+import pytest
+
+import aiehlc_amd as mi
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def _i8(rng, *shape):
+    return rng.integers(-128, 128, size=shape, dtype=np.int8)
+
+
+GEMM_SHAPES = [
+    # M, N, K
+    (1, 16, 16),      # the smallest that runs here: one chunk of one row
+    (1, 17, 17),      # one byte past a chunk in k and in columns
+    (3, 127, 31),     # a skinny tile one column short
+    (16, 129, 255),   # ... and one column over, one byte short of a stage
+    (17, 64, 256),    # one row past the skinny tile, whole stages
+    (63, 65, 257),    # the 64 x 64 tile, one short and one over
+    (64, 64, 100),
+    (130, 70, 515),   # three stages, the last of 3 bytes
+    (5, 40, 4099),    # one tile, 17 stages: split over many workgroups
+    (70, 300, 2050),  # ten tiles, split
+    (300, 700, 200),
+    (1100, 1030, 330),  # more tiles than CUs
+    (2500, 2300, 70),   # large enough for the 128 x 128 tile
+    (9, 33, 65600),   # K >= 2^16: the requant form without the rounding add
+]
+
+
+@pytest.mark.parametrize("M,N,K", GEMM_SHAPES)
+@pytest.mark.parametrize("layout", [mi.B_NN, mi.B_NT])
+def test_gemm_i8_flex(ctx, M, N, K, layout):
+    print(f"[case] flex gemm {M}x{N}x{K} layout {layout} plan {ctx.plan_gemm_i8(M, N, K)}", flush=True)
+    rng = np.random.default_rng(M + 3 * N + 5 * K + layout)
+    A = _i8(rng, M, K)
+    B = _i8(rng, N, K) if layout == mi.B_NT else _i8(rng, K, N)
+    Co = oracle.gemm_i8(A, B, b_nt=layout == mi.B_NT)
+    shift = 10
+    dA, dB = ctx.upload(A), ctx.upload(B)
+    dY, dC, dY2 = ctx.empty((M, N), np.int8), ctx.empty((M, N), np.int32), ctx.empty((M, N), np.int8)
+    for rep in range(3):
+        ctx.copy_h2d(dY, np.full((M, N), 77, np.int8))
+        ctx.copy_h2d(dC, np.full((M, N), 77, np.int32))
+        ctx.gemm_i8_rq(dA, dB, dY, M, N, K, shift, rep == 1, dC, layout)
+        ctx.gemm_i8_rq(dA, dB, dY2, M, N, K, 0, False, None, layout)
+        ctx.wait(60_000)
+        assert np.array_equal(ctx.download(dC), Co), rep
+        assert np.array_equal(ctx.download(dY), oracle.requant(Co, shift, relu=rep == 1)), rep
+        assert np.array_equal(ctx.download(dY2), oracle.requant(Co, 0)), rep
+    for b in (dA, dB, dY, dC, dY2):
+        b.free()
+
+
+@pytest.mark.parametrize("M,N,K,layout", [(5, 40, 1000, mi.B_NN), (70, 90, 300, mi.B_NT), (130, 150, 48, mi.B_NN),
+                                          (33, 100, 2100, mi.B_NT)])
+@pytest.mark.parametrize("off", [1, 3, 8])
+def test_gemm_i8_flex_strided_unaligned(ctx, M, N, K, layout, off):
+    """Operands at byte offset `off` with padded rows, exactly as long as the
+    entry point says (the last row has no padding), results strided too and
+    the padding between result rows left alone."""
+    lda, ldb, ldc = K + off, (K if layout == mi.B_NT else N) + 2 * off, N + off
+    rows_b = N if layout == mi.B_NT else K
+    cols_b = K if layout == mi.B_NT else N
+    rng = np.random.default_rng(M + N + K + off)
+    A, B = _i8(rng, M, K), _i8(rng, rows_b, cols_b)
+    bufA = _i8(rng, off + (M - 1) * lda + K)
+    bufB = _i8(rng, off + (rows_b - 1) * ldb + cols_b)
+    for m in range(M):
+        bufA[off + m * lda: off + m * lda + K] = A[m]
+    for r in range(rows_b):
+        bufB[off + r * ldb: off + r * ldb + cols_b] = B[r]
+    dA, dB = ctx.upload(bufA), ctx.upload(bufB)
+    sentinel = np.full(1 + (M - 1) * ldc + N, -5, np.int32)  # C at a 4-byte offset
+    dC = ctx.upload(sentinel)
+    ctx.gemm_i8_i32(dA.ptr + off, dB.ptr + off, dC.ptr + 4, M, N, K, lda, ldb, ldc, layout)
+    ctx.wait(60_000)
+    got = ctx.download(dC)
+    want = sentinel.copy()
+    Co = oracle.gemm_i8(A, B, b_nt=layout == mi.B_NT)
+    for m in range(M):
+        want[1 + m * ldc: 1 + m * ldc + N] = Co[m]
+    assert np.array_equal(got, want)
+    for b in (dA, dB, dC):
+        b.free()
+
+
+def test_gemm_i8_flex_recorded(ctx):
+    """Split products in a recorded chain (they share the context's workspace
+    and counters), replayed with eager calls between the replays."""
+    M, N, K, K2 = 7, 300, 3000, 1111
+    rng = np.random.default_rng(5)
+    A, B, B2 = _i8(rng, M, K), _i8(rng, K, K2), _i8(rng, K2, N)
+    dA, dB, dB2 = ctx.upload(A), ctx.upload(B), ctx.upload(B2)
+    dH, dY, dE = ctx.empty((M, K2), np.int8), ctx.empty((M, N), np.int8), ctx.empty((M, K2), np.int8)
+    with ctx.record() as g:
+        ctx.gemm_i8_rq(dA, dB, dH, M, K2, K, 11, True)
+        ctx.gemm_i8_rq(dH, dB2, dY, M, N, K2, 10)
+    for rep in range(4):
+        A = _i8(rng, M, K)
+        ctx.copy_h2d(dA, A)
+        g.launch()
+        ctx.gemm_i8_rq(dA, dB, dE, M, K2, K, 9)
+        ctx.wait(60_000)
+        H = oracle.gemm_i8_rq(A, B, 11, True)
+        assert np.array_equal(ctx.download(dH), H), rep
+        assert np.array_equal(ctx.download(dY), oracle.gemm_i8_rq(H, B2, 10)), rep
+        assert np.array_equal(ctx.download(dE), oracle.gemm_i8_rq(A, B, 9)), rep
+    g.destroy()
+    for b in (dA, dB, dB2, dH, dY, dE):
+        b.free()
