@@ -15,12 +15,15 @@
 //                      v_mfma_f32_16x16x32_bf16 (a higher clock than the
 //                      32x32x16 form under the power limit).
 //   gemm_bf16_tile256  256x256x32, 4 waves x (4x4 MFMA 32x32x16), four LDS stages.
-//   gemm_bf16_tile64p  64x64x32 fallback for K % 8 == 0 and an aligned A:
-//                      vector A loads, next k-tile prefetched into registers.
-//   gemm_bf16_tile64   64x64x32 bounds-checked fallback.
+//   gemm_bf16_flex     register-staged 16x128, 64x64 and 128x128 tiles
+//                      (flex_tile.hpp) for every other size and alignment with
+//                      rows of at least 16 bytes, and wherever 256x256 tiles
+//                      are too few; K split over workgroups.
+//   gemm_bf16_tile64   64x64x32, bounds-checked, for rows below 16 bytes.
 // The 256x256 kernels write C through whole-row stores staged in LDS.
 #include <type_traits>
 
+#include "flex_tile.hpp"
 #include "gfx950_ops.hpp"
 #include "miaie_internal.hpp"
 
@@ -28,6 +31,7 @@ namespace {
 
 namespace dev = miaie::dev;
 namespace dbg = miaie::dbg;
+namespace flex = miaie::flex;
 
 // 64-byte LDS rows: chunk c of row r at chunk c ^ swz(r).  gfx950 serves a
 // ds_read_b128 16 lanes at a time from 64 four-byte banks; XOR with row
@@ -613,58 +617,44 @@ __global__ __launch_bounds__(256) void gemm_bf16_tile64(const uint16_t* __restri
   }
 }
 
-// The 64x64 kernel for K % 8 == 0 and a 16-byte aligned A (a ragged M, N
-// or K): A rows are loaded as full vectors and B columns gathered from clamped,
-// always valid addresses, zeroed when written to LDS if outside the matrix,
-// and the next k-tile's loads are issued before this k-tile's LDS reads and
-// MFMAs, so their latency overlaps the MFMAs.
-__global__ __launch_bounds__(256) void gemm_bf16_tile64p(const uint16_t* __restrict__ A,
-                                                         const uint16_t* __restrict__ B,
-                                                         float* __restrict__ C, int M, int N, int K) {
-  __shared__ __attribute__((aligned(16))) int8_t as[64 * 64];
-  __shared__ __attribute__((aligned(16))) int8_t bs[64 * 64];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int fr = lane & 31, fh = lane >> 5;
-  // A: thread -> row tid/4, 8-element chunk tid%4; B: column tid%64, k-chunk tid/64
-  const int row = tid >> 2, ch = tid & 3, col = tid & 63, bch = tid >> 6;
-  // K % 8 == 0: an 8-element k-chunk lies wholly inside or wholly past K; one
-  // past K loads the row's last chunk instead and is zeroed
-  const bool a_in = m0 + row < M, b_in = n0 + col < N;
-  const uint16_t* const a_p = A + (size_t)min(m0 + row, M - 1) * K;
-  const uint16_t* const b_p = B + min(n0 + col, N - 1);
-  auto load = [&](int k0, v4i& va, v4i& vb) {
-    va = MIAIE_LD(reinterpret_cast<const v4i*>(a_p + min(k0 + 8 * ch, K - 8)));
-    const uint16_t* const p = b_p + (size_t)min(k0 + 8 * bch, K - 8) * N;
-    uint16_t tmp[8];
+// Register-staged tiles (flex_tile.hpp): any size and alignment with rows of
+// at least 16 bytes.  grid.x: output tiles, grid.y: the `splits` workgroups
+// that divide a tile's K.  1000^3 (256 tiles of 64x64, 8 stages, bound by the
+// chain of their loads): 9.4 us, 25.1 in a 64x64 kernel with one 32-wide k-step
+// in flight; 256x4096x2048: 13.7 us split in 2, 40.8 on 16 tiles of 256x256.
+template <class G>
+__global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void gemm_bf16_flex(const uint16_t* __restrict__ A,
+                                                         const uint16_t* __restrict__ B, float* __restrict__ C,
+                                                         int M, int N, int K, int8_t* __restrict__ work,
+                                                         uint32_t* __restrict__ counters) {
+  __shared__ __attribute__((aligned(1024))) int8_t lds[G::LDS];
+  __shared__ int flag;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / G::WAVES_N, wn = wave % G::WAVES_N;
+  int tm, tn;
+  dev::tile_coords<4>(blockIdx.x, (M + G::BM - 1) / G::BM, (N + G::BN - 1) / G::BN, tm, tn);
+  const int m0 = tm * G::BM, n0 = tn * G::BN;
+  const int stages = (2 * K + G::KB - 1) / G::KB, splits = gridDim.y, split = blockIdx.y;
+  const int s0 = (int)((long long)stages * split / splits), s1 = (int)((long long)stages * (split + 1) / splits);
+
+  v4f acc[G::NI][G::NJ];
 #pragma unroll
-    for (int t = 0; t < 8; ++t) tmp[t] = MIAIE_LD(p + (size_t)t * N);
-    __builtin_memcpy(&vb, tmp, 16);
-  };
-  v16f acc = v16f{0.f};
-  v4i va, vb;
-  load(0, va, vb);
-  for (int k0 = 0; k0 < K; k0 += 32) {
-    *reinterpret_cast<v4i*>(as + lds_off(row, ch)) = a_in && k0 + 8 * ch < K ? va : v4i{0};
-    *reinterpret_cast<v4i*>(bs + lds_off(col, bch)) = b_in && k0 + 8 * bch < K ? vb : v4i{0};
-    __syncthreads();
-    if (k0 + 32 < K) load(k0 + 32, va, vb);
+  for (int i = 0; i < G::NI; ++i)
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      const v4i af = *reinterpret_cast<const v4i*>(as + lds_off(wm * 32 + fr, 2 * ks + fh));
-      const v4i bf = *reinterpret_cast<const v4i*>(bs + lds_off(wn * 32 + fr, 2 * ks + fh));
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf(bf), as_bf(af), acc, 0, 0, 0);
-    }
-    __syncthreads();
-  }
-  const int m = m0 + wm * 32 + fr;
-  if (m >= M) return;
+    for (int j = 0; j < G::NJ; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+  flex::RowsLoader<G, G::NA> la(reinterpret_cast<const int8_t*>(A), m0, M, (size_t)K * 2, 2 * K, tid);
+  flex::ColsLoader<uint16_t, G, true> lb(reinterpret_cast<const int8_t*>(B), n0, N, (size_t)N * 2, K, tid);
+  flex::tile_loop<uint16_t, G, true>(lds, la, lb, s0, s1, lane, wm, wn, acc);
+  if (splits > 1 &&
+      !flex::split_sum<uint16_t, G>(acc, blockIdx.x, split, splits, work, counters, &flag, tid))
+    return;
+
+  const int fr = lane & 15, fg = lane >> 4;
 #pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    const int n = n0 + wn * 32 + 8 * (e >> 2) + 4 * fh + (e & 3);
-    if (n < N) MIAIE_ST(C + (size_t)m * N + n, acc[e]);
-  }
+  for (int i = 0; i < G::NI; ++i)
+#pragma unroll
+    for (int j = 0; j < G::NJ; ++j)
+      flex::store4(C, N, m0 + wm * G::WM + 16 * i + fr, n0 + wn * G::WN + 16 * j + 4 * fg, M, N, acc[i][j]);
 }
 
 }  // namespace
@@ -675,26 +665,37 @@ int launch_gemm_bf16(miaie_ctx* ctx, const uint16_t* A, const uint16_t* B, float
   // 256x256 kernels: 16-byte aligned operands, per-lane copy offsets of up
   // to 64 rows in 32 bits, and whole tiles, or else the last tile row
   // (column) moved back over its neighbour (dev::tile_origin; N % 8 == 0
-  // keeps B and C rows on 16-byte chunks) when the tiles fill at least half
-  // the CUs (fewer, and the 64x64 kernel's wider grid is the faster one).
+  // keeps B and C rows on 16-byte chunks).
   const long tiles = (long)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-  const bool whole = M % BM == 0 && N % BN == 0;
-  const bool overlap = M >= BM && N >= BN && N % 8 == 0 && 2 * tiles >= ctx->cus;
-  const bool big = (whole || overlap) && K % BK == 0 && aligned(A, 16) && aligned(B, 16) && aligned(C, 16) &&
-                   K < (1 << 24) && N < (1 << 24);
-  if (big && K % (2 * BK) == 0) {
-    return check_launch(ctx, launch<gemm_bf16_pair16>(ctx->device, dim3(tiles), dim3(256), 0, ctx->stream, A, B, C, M, N, K),
-                        "gemm_bf16_pair16");
-  }
-  if (big) {
+  const bool big = M >= BM && N >= BN && N % 8 == 0 && K % BK == 0 && aligned(A, 16) && aligned(B, 16) &&
+                   aligned(C, 16) && K < (1 << 24) && N < (1 << 24);
+  // Register-staged tiles: rows of at least 16 bytes, and 32-bit offsets
+  // within a tile.
+  const bool flexible = K >= 8 && N >= 8 && K < (1 << 24) && N < (1 << 24);
+  const dim3 grid((N + 63) / 64, (M + 63) / 64);
+  flex::Plan f;
+  if (flexible) f = flex::plan(M, N, 2l * K, 1.0, ctx->cus, true, ctx->work_bytes);
+  // Where both apply, the one estimated faster: a round of 256x256 tiles takes
+  // about 3 us and 0.0185 us per k (1024^3, 16 tiles: 23.6 us, 8.5 on 256 of
+  // 64x64; 2048x4096x2048, 128 tiles: 43.1 us, as on 512 of 128x128).
+  const double big_us = 3.0 + (double)((tiles + ctx->cus - 1) / ctx->cus) * (3.0 + 0.0185 * K);
+  if (big && (!flexible || big_us <= f.us)) {
+    if (K % (2 * BK) == 0)
+      return check_launch(ctx, launch<gemm_bf16_pair16>(ctx->device, dim3(tiles), dim3(256), 0, ctx->stream, A, B, C, M, N, K),
+                          "gemm_bf16_pair16");
     return check_launch(ctx, launch<gemm_bf16_tile256>(ctx->device, dim3(tiles), dim3(256), 0, ctx->stream, A, B, C, M, N, K),
                         "gemm_bf16_tile256");
   }
-  dim3 grid((N + 63) / 64, (M + 63) / 64);
   if (grid.y > 65535) return fail(ctx, MIAIE_EINVAL, "gemm_bf16: M too large for the 64x64 fallback");
-  if (K % 8 == 0 && aligned(A, 16)) {
-    return check_launch(ctx, launch<gemm_bf16_tile64p>(ctx->device, grid, dim3(256), 0, ctx->stream, A, B, C, M, N, K),
-                        "gemm_bf16_tile64p");
+  if (flexible) {
+    if (f.splits > 1 && !may_split(ctx)) f = flex::plan(M, N, 2l * K, 1.0, ctx->cus, false, 0);
+    hipError_t e = hipSuccess;
+    flex::with_geom(f, [&](auto g) {
+      using G = typename decltype(g)::type;
+      e = launch<gemm_bf16_flex<G>>(ctx->device, dim3((unsigned)f.tiles, (unsigned)f.splits), dim3(256), 0, ctx->stream,
+                                    A, B, C, M, N, K, static_cast<int8_t*>(ctx->work), ctx->counters);
+    });
+    return check_launch(ctx, e, "gemm_bf16_flex");
   }
   return check_launch(ctx, launch<gemm_bf16_tile64>(ctx->device, grid, dim3(256), 0, ctx->stream, A, B, C, M, N, K),
                       "gemm_bf16_tile64");

@@ -1,4 +1,4 @@
-"""The register-staged tiles (csrc/flex_tile.hpp): int8 GEMM for every shape,
+"""The register-staged tiles (csrc/flex_tile.hpp): int8 and bf16 GEMM for every shape,
 stride and alignment the pipelined kernels do not take, with K split over
 workgroups where tiles are few.  Sizes at the edges of the tiles (16 x 128,
 64 x 64, 128 x 128), of the 16-byte chunks and of the 256-byte stages; each call
@@ -8,6 +8,7 @@ import pytest
 
 import aiehlc_amd as mi
 import oracle
+from aiehlc_amd import synth
 
 pytestmark = pytest.mark.gpu
 
@@ -115,4 +116,90 @@ def test_gemm_i8_flex_recorded(ctx):
         assert np.array_equal(ctx.download(dE), oracle.gemm_i8_rq(A, B, 9)), rep
     g.destroy()
     for b in (dA, dB, dB2, dH, dY, dE):
+        b.free()
+
+
+# bf16 products are exact in fp32; each of the K additions is off by at most
+# 2^-24 / 2 of a partial sum, whose size stays below 6 times the results' rms
+# (partial sums of N(0, 1) terms scaled to it, over at most 6e6 results)
+def _bf16_bar(K):
+    return 6 * max(K, 32) * 2.0**-25
+
+
+BF16_SHAPES = [
+    (1, 8, 8),        # the smallest that runs here: one chunk of one row
+    (1, 9, 9),        # a value past a chunk
+    (16, 127, 127),   # skinny tile, one column short, a value short of a stage
+    (17, 129, 128),
+    (63, 65, 129),
+    (64, 64, 33),
+    (4, 40, 4100),    # one tile, 33 stages: split
+    (130, 270, 1030),  # split, ragged
+    (1024, 512, 512),  # whole 256x256 tiles, but few
+    (1000, 1000, 100),
+    (2500, 2300, 40),  # large enough for the 128x128 tile
+]
+
+
+@pytest.mark.parametrize("M,N,K", BF16_SHAPES)
+def test_gemm_bf16_flex(ctx, M, N, K):
+    print(f"[case] flex bf16 {M}x{N}x{K}", flush=True)
+    A = synth.bf16_normal((M, K), 1, 1.0 / np.sqrt(K))
+    B = synth.bf16_normal((K, N), 2, 1.0)
+    # what lies past the operands' ends must not matter: they sit between NaNs
+    nan = np.full(64, 0x7FC0, np.uint16)
+    dA, dB = ctx.upload(np.concatenate([nan, A.ravel(), nan])), ctx.upload(np.concatenate([nan, B.ravel(), nan]))
+    R = oracle.gemm_bf16(A, B, f64=True)
+    dC = ctx.empty((M, N), np.float32)
+    first = None
+    for rep in range(3):
+        ctx.copy_h2d(dC, np.full((M, N), np.nan, np.float32))
+        ctx.gemm_bf16_f32(dA.ptr + 128, dB.ptr + 128, dC, M, N, K)
+        ctx.wait(60_000)
+        C = ctx.download(dC)
+        err = np.abs(C.astype(np.float64) - R).max() / np.sqrt(np.mean(R * R))
+        assert err <= _bf16_bar(K), (rep, err)
+        # the order of arrival of the splits does not matter
+        assert first is None or np.array_equal(C, first), rep
+        first = C
+    for b in (dA, dB, dC):
+        b.free()
+
+
+def test_gemm_bf16_flex_nan_stays_in_its_row_and_column(ctx):
+    """A NaN or infinity in one row of A (column of B) reaches that row
+    (column) of C alone, K and N ragged."""
+    M, N, K = 70, 75, 150
+    A, B = synth.bf16_normal((M, K), 3, 0.1), synth.bf16_normal((K, N), 4, 1.0)
+    A[11, K - 1] = 0x7FC0  # NaN
+    B[K - 1, 66] = 0x7F80  # inf
+    dA, dB, dC = ctx.upload(A), ctx.upload(B), ctx.empty((M, N), np.float32)
+    ctx.gemm_bf16_f32(dA, dB, dC, M, N, K)
+    ctx.wait(60_000)
+    bad = ~np.isfinite(ctx.download(dC))
+    want = np.zeros((M, N), bool)
+    want[11, :] = True
+    want[:, 66] = True
+    assert np.array_equal(bad, want)
+    for b in (dA, dB, dC):
+        b.free()
+
+
+@pytest.mark.parametrize("K", [32, 64, 96, 128, 192, 256, 320, 384, 448, 512, 576, 1088, 2112])
+def test_gemm_bf16_256_tiles_k_sweep(ctx, K):
+    """Every k-tile count of the 256x256 kernels' prologue and tail, planned
+    for one CU so that they are the choice."""
+    M, N = 512, 256
+    A, B = synth.bf16_normal((M, K), 5, 1.0 / np.sqrt(K)), synth.bf16_normal((K, N), 6, 1.0)
+    dA, dB, dC = ctx.upload(A), ctx.upload(B), ctx.empty((M, N), np.float32)
+    prev = ctx.plan_set_cus(1)
+    try:
+        ctx.gemm_bf16_f32(dA, dB, dC, M, N, K)
+        ctx.wait(60_000)
+    finally:
+        ctx.plan_set_cus(prev)
+    R = oracle.gemm_bf16(A, B, f64=True)
+    err = np.abs(ctx.download(dC).astype(np.float64) - R).max() / np.sqrt(np.mean(R * R))
+    assert err <= _bf16_bar(K), err
+    for b in (dA, dB, dC):
         b.free()
