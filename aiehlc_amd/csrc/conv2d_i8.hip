@@ -7,8 +7,11 @@
 // benchmark's: zero padding, stride, int32 accumulation, then
 // y = sat_int8((acc + 2^(s_c-1)) >> s_c) per output channel c.
 //
+// Kernels: the row-block kernels (conv2d_i8_rows.hpp), conv2d_i8_taps,
+// conv2d_i8_igemm, and conv2d_i8_flex for every other shape.
+//
 // GEMM view: rows = output pixels (n, ho, wo), columns = output channels,
-// k = (r, s, ci).  A workgroup owns 64 consecutive pixels x 64 channels.
+// k = (r, s, ci).  A workgroup of conv2d_i8_igemm owns 64 consecutive pixels x 64 channels.
 // Each of its 4 waves takes every 4th k-step of 32 (one (r, s, ci-block)),
 // loading X and W fragments straight from global memory in MFMA operand
 // layout (W rows are k-contiguous in OHWI; X pixels are ci-contiguous in
@@ -25,10 +28,13 @@
 #include <algorithm>
 
 #include "conv2d_i8_rows.hpp"
+#include "flex_tile.hpp"
 #include "gfx950_ops.hpp"
 #include "miaie_internal.hpp"
 
 namespace {
+
+namespace flex = miaie::flex;
 
 __device__ __forceinline__ int requant1(int acc, int s) {
   int q = s ? (acc >> s) + ((acc >> (s - 1)) & 1) : acc;
@@ -430,7 +436,196 @@ __global__ __launch_bounds__(256) void conv2d_i8_splitk_reduce(const int32_t* __
   MIAIE_ST(reinterpret_cast<uint4*>(Y + e), make_uint4(out[0], out[1], out[2], out[3]));
 }
 
-// Any-shape fallback: one thread per output element.
+// ------------------------------------------------------- register-staged kernel
+// Any shape, as an implicit GEMM on the register-staged tiles (flex_tile.hpp):
+// rows are output pixels, columns output channels.  For one filter row r the
+// S * Cin input bytes under the filter are one contiguous run of the image row
+// hi = ho * stride - pad + r, and so are the weights' (r, :, :): k is taken as R such
+// runs, each padded to whole 16-byte chunks (CPR per run).  The weights' chunks
+// are zero past their run, so what the pixels' hold there does not matter
+// (a neighbour's bytes); bytes outside the image row are zeroed.
+struct RunShape {
+  int H, Wd, Cin, R, Ho, Wo, stride, pad;
+  int SC, CPR;                    // bytes per run (S * Cin), 16-byte chunks per run
+  uint32_t cpr_inv, wo_inv, ho_inv;  // see div_small
+};
+// x / d with inv = floor(2^32 / d) + 1: exact for x * d < 2^32 and d > 1
+__device__ __forceinline__ int div_small(int x, int d, uint32_t inv) { return d == 1 ? x : (int)__umulhi((uint32_t)x, inv); }
+
+// chunk q = s * CH + ch of the k runs of pixels p0 + r0 + RPP i.  Byte
+// offsets are 32-bit (the launcher keeps X below 2^31 bytes).
+template <class G, int NL>
+struct PixelLoader {
+  const int8_t* X;
+  const RunShape& k;
+  int last;        // last offset a 16-byte load may start at
+  int r0, ch;
+  int hi0[NL];     // first input row under the filter (negative in the padding)
+  int xb[NL];      // first byte of the run within its row (likewise)
+  int at0[NL];     // its offset in X
+  v4i v[NL];
+  int keep[NL];    // valid bytes [keep & 255, keep >> 8)
+  int moved[NL];   // distance a load was moved to stay inside X
+  bool edge, shift;
+  __device__ __forceinline__ PixelLoader(const int8_t* X_, const RunShape& k_, int total, int p0, int P, int tid)
+      : X(X_), k(k_), last(total - 16), r0(tid / G::CH), ch(tid % G::CH), edge(false), shift(false) {
+    // one pixel divided out, the thread's others from there (RPP i further,
+    // at most BM rows and columns: small quotients)
+    const uint32_t p = (uint32_t)min(p0 + r0, P - 1), t = p / (uint32_t)k.Wo;
+    const int wo0 = (int)(p - t * k.Wo), n0 = (int)(t / (uint32_t)k.Ho), ho0 = (int)t - n0 * k.Ho;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int x = wo0 + min(G::RPP * i, P - 1 - (int)p);  // (pixels past the last repeat it)
+      const int dh = k.Wo > G::BM ? (int)(x >= k.Wo) : div_small(x, k.Wo, k.wo_inv);
+      const int y = ho0 + dh, dn = k.Ho > G::BM ? (int)(y >= k.Ho) : div_small(y, k.Ho, k.ho_inv);
+      hi0[i] = (y - dn * k.Ho) * k.stride - k.pad;
+      xb[i] = ((x - dh * k.Wo) * k.stride - k.pad) * k.Cin;
+      at0[i] = ((n0 + dn) * k.H + hi0[i]) * (k.Wd * k.Cin) + xb[i];
+    }
+  }
+  __device__ __forceinline__ void load(int s) {
+    const int q = s * G::CH + ch;
+    int r = div_small(q, k.CPR, k.cpr_inv), c = q - r * k.CPR;
+    if (r >= k.R) r = c = 0;  // past the last run (zero weights)
+    const int row_bytes = k.Wd * k.Cin, step = r * row_bytes + 16 * c;
+    bool e = false, m = false;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      // (a row outside the image is loaded from wherever the offset points,
+      // moved inside X, and zeroed)
+      const int at = at0[i] + step, from = min(max(at, 0), last), b = xb[i] + 16 * c;
+      v[i] = MIAIE_LD(reinterpret_cast<const flex::Any16*>(X + (uint32_t)from)).v;
+      const int lo = min(max(-b, 0), 16);
+      const int up = (unsigned)(hi0[i] + r) < (unsigned)k.H ? min(max(row_bytes - b, 0), 16) : 0;
+      moved[i] = at - from;
+      keep[i] = lo | up << 8;
+      e |= keep[i] != (16 << 8);
+      m |= moved[i] != 0;
+    }
+    edge = __builtin_amdgcn_ballot_w64(e) != 0;
+    shift = __builtin_amdgcn_ballot_w64(m) != 0;
+  }
+  __device__ __forceinline__ void put(int, int8_t* lds) {
+    if (shift) {
+#pragma unroll
+      for (int i = 0; i < NL; ++i)
+        v[i] = flex::shl_bytes(flex::shr_bytes(v[i], min(max(moved[i], 0), 16)), min(max(-moved[i], 0), 16));
+    }
+    if (edge) {
+#pragma unroll
+      for (int i = 0; i < NL; ++i) v[i] = v[i] & flex::byte_mask(keep[i] & 255, keep[i] >> 8);
+    }
+#pragma unroll
+    for (int i = 0; i < NL; ++i) *reinterpret_cast<v4i*>(lds + flex::row_off(G::KB, r0 + G::RPP * i, ch)) = v[i];
+  }
+};
+
+// the same chunks of the weights of channels co0 + r0 + RPP i, zero past
+// their run
+template <class G, int NL>
+struct WeightLoader {
+  const int8_t* W;
+  const RunShape& k;
+  int last, r0, ch, valid;
+  int at0[NL];
+  v4i v[NL];
+  int moved[NL];
+  bool shift;
+  __device__ __forceinline__ WeightLoader(const int8_t* W_, const RunShape& k_, int co0, int Cout, int tid)
+      : W(W_), k(k_), last(Cout * k_.R * k_.SC - 16), r0(tid / G::CH), ch(tid % G::CH), valid(0), shift(false) {
+#pragma unroll
+    for (int i = 0; i < NL; ++i) at0[i] = min(co0 + r0 + G::RPP * i, Cout - 1) * (k.R * k.SC);
+  }
+  __device__ __forceinline__ void load(int s) {
+    const int q = s * G::CH + ch;
+    int r = div_small(q, k.CPR, k.cpr_inv), c = q - r * k.CPR;
+    valid = r < k.R ? min(k.SC - 16 * c, 16) : 0;
+    if (r >= k.R) r = c = 0;
+    const int step = r * k.SC + 16 * c;
+    bool m = false;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int at = at0[i] + step, from = min(at, last);
+      v[i] = MIAIE_LD(reinterpret_cast<const flex::Any16*>(W + (uint32_t)from)).v;
+      moved[i] = at - from;
+      m |= moved[i] != 0;
+    }
+    shift = __builtin_amdgcn_ballot_w64(m) != 0;
+  }
+  __device__ __forceinline__ void put(int, int8_t* lds) {
+    if (shift) {
+#pragma unroll
+      for (int i = 0; i < NL; ++i) v[i] = flex::shr_bytes(v[i], min(moved[i], 16));
+    }
+    const v4i mask = flex::byte_mask(0, valid);
+#pragma unroll
+    for (int i = 0; i < NL; ++i) *reinterpret_cast<v4i*>(lds + flex::row_off(G::KB, r0 + G::RPP * i, ch)) = v[i] & mask;
+  }
+};
+
+// Bound by its vector instructions: with few channels a workgroup has one
+// stage, and the pixels' addresses, masks and the requantize outweigh the
+// MFMAs.  8x224x224x3 -> 64, 7x7, stride 2 (1568 tiles of 64x64, one stage of
+// 224 bytes): 12.8 us, 919 with one thread per output; 8x48x48x96 -> 146, 5x5:
+// 29 us.
+template <class G>
+__global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void conv2d_i8_flex(const int8_t* __restrict__ X, const int8_t* __restrict__ W,
+                                                         const uint8_t* __restrict__ shifts, int8_t* __restrict__ Y,
+                                                         RunShape k, int x_bytes, int P, int Cout,
+                                                         int8_t* __restrict__ work, uint32_t* __restrict__ counters) {
+  __shared__ __attribute__((aligned(1024))) int8_t lds[G::LDS];
+  __shared__ int flag;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / G::WAVES_N, wn = wave % G::WAVES_N;
+  int tm, tn;
+  miaie::dev::tile_coords<4>(blockIdx.x, (P + G::BM - 1) / G::BM, (Cout + G::BN - 1) / G::BN, tm, tn);
+  const int p0 = tm * G::BM, co0 = tn * G::BN;
+  const int stages = (k.R * k.CPR + G::CH - 1) / G::CH, splits = gridDim.y, split = blockIdx.y;
+  const int s0 = (int)((long long)stages * split / splits), s1 = (int)((long long)stages * (split + 1) / splits);
+
+  v4i acc[G::NI][G::NJ];
+#pragma unroll
+  for (int i = 0; i < G::NI; ++i)
+#pragma unroll
+    for (int j = 0; j < G::NJ; ++j) acc[i][j] = v4i{0};
+  // this lane's channels' shifts, in flight during the main loop
+  const int fr = lane & 15, fg = lane >> 4;
+  int sh[G::NJ][4];
+#pragma unroll
+  for (int j = 0; j < G::NJ; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      sh[j][e] = MIAIE_LD(shifts + min(co0 + wn * G::WN + 16 * j + 4 * fg + e, Cout - 1));
+  PixelLoader<G, G::NA> la(X, k, x_bytes, p0, P, tid);
+  WeightLoader<G, G::NB> lb(W, k, co0, Cout, tid);
+  flex::tile_loop<int8_t, G, false>(lds, la, lb, s0, s1, lane, wm, wn, acc);
+  if (splits > 1 &&
+      !flex::split_sum<int8_t, G>(acc, blockIdx.x, split, splits, work, counters, &flag, tid))
+    return;
+
+#pragma unroll
+  for (int j = 0; j < G::NJ; ++j) {
+    const int nl = wn * G::WN + 16 * j + 4 * fg;
+#pragma unroll
+    for (int i = 0; i < G::NI; ++i) {
+      uint32_t y = 0;
+      if (k.R * k.SC < (1 << 16)) {  // |acc| < 2^30: room for the rounding term
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          y |= (uint32_t)(min(max((acc[i][j][e] + (int)((1u << sh[j][e]) >> 1)) >> sh[j][e], -128), 127) & 0xFF) << (8 * e);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y |= (uint32_t)(requant1(acc[i][j][e], sh[j][e]) & 0xFF) << (8 * e);
+      }
+      *reinterpret_cast<uint32_t*>(lds + (wm * G::WM + 16 * i + fr) * G::YP + nl) = y;
+    }
+  }
+  __syncthreads();
+  flex::store_y<G>(lds, Y, Cout, p0, co0, P, Cout, tid);
+}
+
+// Operands of fewer than 16 bytes, and above 2^31: one thread per output
+// element.
 __global__ __launch_bounds__(256) void conv2d_i8_direct(const int8_t* __restrict__ X, const int8_t* __restrict__ W,
                                                         const uint8_t* __restrict__ shifts, int8_t* __restrict__ Y,
                                                         int N, int H, int Wd, int Cin, int Cout, int R, int S,
@@ -604,6 +799,37 @@ int conv2d_kernel_for(int N, int H, int Wd, int Cin, int Cout, int R, int S, int
   return MIAIE_CONV_DIRECT;
 }
 
+// The register-staged kernel: X and W of at least 16 bytes (one load) and
+// below 2^31, with the padding around X included (offsets of runs that start
+// in it are computed before they are moved inside).
+static bool flex_ok(int N, int H, int Wd, int Cin, int Cout, int R, int S, int pad, size_t P) {
+  const size_t sc = (size_t)S * Cin, cpr = (sc + 15) / 16, lim = ((size_t)1 << 31) - (1 << 12);
+  const size_t row = ((size_t)Wd + 2 * (size_t)pad) * Cin + 16;
+  return (size_t)N * H * Wd * Cin >= 16 && (size_t)Cout * R * sc >= 16 && row < lim &&
+         ((size_t)N * H + 2 * (size_t)pad + R) * row < lim && (size_t)Cout * R * sc < lim && P < lim &&
+         (R * cpr + 64) * cpr < ((size_t)1 << 32);
+}
+
+static int launch_flex(miaie_ctx* ctx, const int8_t* X, const int8_t* W, const uint8_t* shifts, int8_t* Y, int N, int H,
+                       int Wd, int Cin, int Cout, int R, int S, int stride, int pad, int Ho, int Wo) {
+  RunShape k{H, Wd, Cin, R, Ho, Wo, stride, pad, S * Cin, (S * Cin + 15) / 16, 0, 0, 0};
+  auto inverse = [](int d) { return (uint32_t)(((uint64_t)1 << 32) / (uint64_t)d + 1); };
+  k.cpr_inv = inverse(k.CPR);
+  k.wo_inv = inverse(Wo);
+  k.ho_inv = inverse(Ho);
+  const long P = (long)N * Ho * Wo;
+  flex::Plan f = flex::plan(P, Cout, 16l * R * k.CPR, 1.5, ctx->cus, true, ctx->work_bytes);
+  if (f.splits > 1 && !may_split(ctx)) f = flex::plan(P, Cout, 16l * R * k.CPR, 1.5, ctx->cus, false, 0);
+  hipError_t e = hipSuccess;
+  flex::with_geom(f, [&](auto g) {
+    using G = typename decltype(g)::type;
+    e = launch<conv2d_i8_flex<G>>(ctx->device, dim3((unsigned)f.tiles, (unsigned)f.splits), dim3(256), 0, ctx->stream, X,
+                                  W, shifts, Y, k, N * H * Wd * Cin, (int)P, Cout, static_cast<int8_t*>(ctx->work),
+                                  ctx->counters);
+  });
+  return check_launch(ctx, e, "conv2d_i8_flex");
+}
+
 int launch_conv2d_i8(miaie_ctx* ctx, const int8_t* X, const int8_t* W, const uint8_t* shifts, int8_t* Y,
                      int N, int H, int Wd, int Cin, int Cout, int R, int S, int stride, int pad) {
   const int Ho = (H + 2 * pad - R) / stride + 1;
@@ -662,7 +888,15 @@ int launch_conv2d_i8(miaie_ctx* ctx, const int8_t* X, const int8_t* W, const uin
                                                                stride, pad, Ho, Wo, 1);
     return check_launch(ctx, e, "conv2d_i8_taps");
   }
-  if (kernel == MIAIE_CONV_IGEMM) {
+  // Three 64x64 tiles per CU or more: the register-staged kernel in place of
+  // the implicit GEMM on fragments from memory, which is the faster one below
+  // that (its workgroups start sooner), and the slower one above, where each
+  // fragment load touches 32 lines (4x112x112x96->256: 38.1 against 33.2 us;
+  // 8x64x64x160->512 1x1: 25.9 against 15.5; 2x56x56x64->64 stride 2, 25 tiles:
+  // 4.7 against 6.8).
+  const bool big = ((P + 63) / 64) * (size_t)((Cout + 63) / 64) >= 3 * (size_t)ctx->cus;
+  const bool flex = flex_ok(N, H, Wd, Cin, Cout, R, S, pad, P);
+  if (kernel == MIAIE_CONV_IGEMM && !(big && flex)) {
     const unsigned pxb = (unsigned)((P + PIX - 1) / PIX), chb = (unsigned)(Cout / COB);
     const int ks = conv_ksplit((size_t)pxb * chb, R * S * (Cin / 32), 4 * BATCH, P * Cout, ctx->cus, ctx->work_bytes);
     if (ks > 1) {
@@ -681,6 +915,8 @@ int launch_conv2d_i8(miaie_ctx* ctx, const int8_t* X, const int8_t* W, const uin
                                                         Ho, Wo, 1);
     return check_launch(ctx, e, "conv2d_i8_igemm");
   }
+  if (flex) return launch_flex(ctx, X, W, shifts, Y, N, H, Wd, Cin, Cout, R, S, stride, pad, Ho, Wo);
+  // operands below 16 or above 2^31 bytes
   const size_t total = P * Cout;
   const size_t blocks = (total + 255) / 256;
   if (blocks >= ((size_t)1 << 31)) return fail(ctx, MIAIE_EINVAL, "conv2d: output too large for the direct kernel");

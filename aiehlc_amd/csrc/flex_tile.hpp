@@ -87,31 +87,32 @@ struct Plan {
 // worst).  A tile of 32 x 128 was never more than 2% better than these three.
 // `cost`: stage cost relative to the int8 GEMM's (conv 1.5: its loads compute
 // their addresses).
-inline Plan plan(long M, long N, long k_bytes, double cost, int cus, bool can_split, size_t work_bytes) {
-  struct Tile {
-    int bm, bn, kb;
-    double t0, latency, wg, stage, sum, sum_split;
-  };
-  static constexpr Tile kTiles[] = {
-      {Skinny::BM, Skinny::BN, Skinny::KB, 1.7, 0.95, 0.90, 0.80, 1.6, 0.15},
-      {Small::BM, Small::BN, Small::KB, 2.4, 0.84, 0.55, 0.50, 1.5, 0.26},
-      {Large::BM, Large::BN, Large::KB, 3.5, 0.95, 1.20, 0.60, 1.5, 1.00},
-  };
+// (No divisions: this runs on the host for every call.)
+template <class G>
+inline void consider(Plan& best, double t0, double latency, double wg, double stage, double sum, double sum_split,
+                     long M, long N, long k_bytes, double cost, int cus, double per_cu, bool can_split,
+                     size_t work_bytes) {
   static constexpr int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16};
-  Plan best;
-  for (const Tile& t : kTiles) {
-    const long tiles = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn), stages = (k_bytes + t.kb - 1) / t.kb;
-    const size_t slot = (size_t)tiles * t.bm * t.bn * sizeof(int32_t);
-    for (int s : kSplits) {
-      // (more than four workgroups per CU never split)
-      if (s > 1 && (!can_split || s > stages || tiles * s > 4l * cus || tiles > MIAIE_CTX_COUNTERS || slot * s > work_bytes))
-        break;
-      const double n = (double)((stages + s - 1) / s), rounds = (double)((tiles * s + cus - 1) / cus);
-      const double us = t.t0 + std::max(t.latency * cost * n, rounds * (t.wg + t.stage * cost * n)) +
-                        (s > 1 ? t.sum + t.sum_split * s : 0.0);
-      if (best.bm == 0 || us < best.us) best = Plan{t.bm, t.bn, s, tiles, us};
-    }
+  static constexpr double kInverse[] = {1.0, 1.0 / 2, 1.0 / 3, 1.0 / 4, 1.0 / 6, 1.0 / 8, 1.0 / 12, 1.0 / 16};
+  const long tiles = ((M + G::BM - 1) / G::BM) * ((N + G::BN - 1) / G::BN), stages = (k_bytes + G::KB - 1) / G::KB;
+  const size_t slot = (size_t)tiles * G::BM * G::BN * sizeof(int32_t);
+  auto up = [](double x) { return (double)(long)(x + (1.0 - 1e-6)); };  // rounded up
+  for (int i = 0; i < 8; ++i) {
+    const int s = kSplits[i];
+    // (more than four workgroups per CU never split)
+    if (s > 1 && (!can_split || s > stages || tiles * s > 4l * cus || tiles > MIAIE_CTX_COUNTERS || slot * s > work_bytes))
+      return;
+    const double n = up((double)stages * kInverse[i]), rounds = up((double)(tiles * s) * per_cu);
+    const double us = t0 + std::max(latency * cost * n, rounds * (wg + stage * cost * n)) + (s > 1 ? sum + sum_split * s : 0.0);
+    if (best.bm == 0 || us < best.us) best = Plan{G::BM, G::BN, s, tiles, us};
   }
+}
+inline Plan plan(long M, long N, long k_bytes, double cost, int cus, bool can_split, size_t work_bytes) {
+  Plan best;
+  const double per_cu = 1.0 / cus;
+  consider<Skinny>(best, 1.7, 0.95, 0.90, 0.80, 1.6, 0.15, M, N, k_bytes, cost, cus, per_cu, can_split, work_bytes);
+  consider<Small>(best, 2.4, 0.84, 0.55, 0.50, 1.5, 0.26, M, N, k_bytes, cost, cus, per_cu, can_split, work_bytes);
+  consider<Large>(best, 3.5, 0.95, 1.20, 0.60, 1.5, 1.00, M, N, k_bytes, cost, cus, per_cu, can_split, work_bytes);
   return best;
 }
 

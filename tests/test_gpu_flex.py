@@ -1,4 +1,4 @@
-"""The register-staged tiles (csrc/flex_tile.hpp): int8 and bf16 GEMM for every shape,
+"""The register-staged tiles (csrc/flex_tile.hpp): int8 and bf16 GEMM and conv for every shape,
 stride and alignment the pipelined kernels do not take, with K split over
 workgroups where tiles are few.  Sizes at the edges of the tiles (16 x 128,
 64 x 64, 128 x 128), of the 16-byte chunks and of the 256-byte stages; each call
@@ -202,4 +202,54 @@ def test_gemm_bf16_256_tiles_k_sweep(ctx, K):
     err = np.abs(ctx.download(dC).astype(np.float64) - R).max() / np.sqrt(np.mean(R * R))
     assert err <= _bf16_bar(K), err
     for b in (dA, dB, dC):
+        b.free()
+
+
+CONV_SHAPES = [
+    # N, H, W, Cin, Cout, R, S, stride, pad
+    (1, 4, 4, 1, 1, 1, 1, 1, 0),      # 16 bytes of X; W (1 byte) too small: one thread per output
+    (1, 4, 4, 1, 16, 1, 1, 1, 0),     # the smallest operands that run here
+    (2, 9, 11, 3, 64, 7, 7, 2, 3),    # a stem: runs of 21 bytes, pads on every side
+    (1, 5, 5, 5, 3, 3, 3, 1, 1),      # pixels fewer than a tile, 3 channels
+    (3, 7, 1, 16, 65, 3, 1, 1, 1),    # one column, R != S, one channel past a tile
+    (2, 1, 30, 6, 20, 1, 5, 1, 2),    # padding rows only above and below a single row
+    (1, 3, 3, 30, 40, 3, 3, 1, 4),    # padding wider than the filter: runs wholly outside
+    (5, 6, 7, 33, 17, 3, 3, 3, 1),    # stride 3
+    (1, 70, 130, 17, 66, 3, 3, 1, 1),  # rows longer than a pixel tile
+    (40, 3, 2, 8, 24, 2, 2, 1, 0),    # many images within one pixel tile (two output columns, one row... 2 x 1)
+    (1, 13, 13, 130, 70, 5, 5, 1, 2),  # k of 5 runs of 650 bytes: stages across runs, split
+    (1, 3, 3, 7300, 5, 3, 3, 1, 1),   # k >= 2^16: the requant form without the rounding add
+    (4, 64, 64, 3, 130, 3, 3, 1, 1),  # 256 x 2 tiles: 128 x 128
+    (8, 96, 96, 32, 192, 1, 1, 1, 0),  # a large grid of the implicit-GEMM shapes
+]
+
+
+@pytest.mark.parametrize("shape", CONV_SHAPES)
+@pytest.mark.parametrize("off", [0, 5])
+def test_conv2d_i8_flex(ctx, shape, off):
+    """Bit-exact against the oracle, shifts over [0, 31], operands at byte
+    offset `off` of their buffers, three calls in a row (split sums leave their
+    counters for the next launch)."""
+    N, H, W, Cin, Cout, R, S, stride, pad = shape
+    print(f"[case] flex conv {shape} off {off}", flush=True)
+    rng = np.random.default_rng(sum(shape) + off)
+    X, Wt = _i8(rng, N, H, W, Cin), _i8(rng, Cout, R, S, Cin)
+    if Cin == 7300:
+        X[:], Wt[:] = -128, -128
+    sh = rng.integers(0, 32, size=Cout, dtype=np.uint8) if sum(shape) % 2 else rng.integers(8, 13, size=Cout, dtype=np.uint8)
+    Ho, Wo = (H + 2 * pad - R) // stride + 1, (W + 2 * pad - S) // stride + 1
+    lead = _i8(rng, off)  # exactly as long as the operands: nothing behind them
+    dX = ctx.upload(np.concatenate([lead, X.ravel()]))
+    dW = ctx.upload(np.concatenate([lead, Wt.ravel()]))
+    dS = ctx.upload(sh)
+    dY = ctx.empty((off + N * Ho * Wo * Cout + 16,), np.int8)
+    want = oracle.conv2d_nhwc_i8(X, Wt, sh, stride, pad).ravel()
+    for rep in range(3):
+        ctx.copy_h2d(dY, np.full(dY.nbytes, 77, np.int8))
+        ctx.conv2d_i8_nhwc(dX.ptr + off, dW.ptr + off, dS, dY.ptr + off, N, H, W, Cin, Cout, R, S, stride, pad)
+        ctx.wait(60_000)
+        got = ctx.download(dY)
+        assert np.array_equal(got[off:-16], want), rep
+        assert (got[:off] == 77).all() and (got[-16:] == 77).all(), rep
+    for b in (dX, dW, dS, dY):
         b.free()
