@@ -154,7 +154,7 @@ __global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void gemm_i8_flex(const i
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / G::WAVES_N, wn = wave % G::WAVES_N;
   int tm, tn;
-  dev::tile_coords<4>(blockIdx.x, (M + G::BM - 1) / G::BM, (N + G::BN - 1) / G::BN, tm, tn);
+  flex::tile_index<!B_NT && G::BN == 64>((M + G::BM - 1) / G::BM, (N + G::BN - 1) / G::BN, tm, tn);
   const int m0 = tm * G::BM, n0 = tn * G::BN;
   const int stages = (K + G::KB - 1) / G::KB, splits = gridDim.y, split = blockIdx.y;
   const int s0 = (int)((long long)stages * split / splits), s1 = (int)((long long)stages * (split + 1) / splits);

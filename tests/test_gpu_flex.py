@@ -32,6 +32,7 @@ GEMM_SHAPES = [
     (300, 700, 200),
     (1100, 1030, 330),  # more tiles than CUs
     (2500, 2300, 70),   # large enough for the 128 x 128 tile
+    (60, 2100, 520),  # one row of 64 x 64 tiles, 33: two paired groups of 16 and one alone
     (9, 33, 65600),   # K >= 2^16: the requant form without the rounding add
 ]
 
