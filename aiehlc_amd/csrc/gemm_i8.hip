@@ -319,6 +319,7 @@ struct TileChoice {
 constexpr TileChoice kTiles[] = {{256, 256, 1.0}, {256, 128, 0.55}, {128, 128, 0.35}};
 
 struct PipePlan {
+  double cost = 0;  // units of one 256x256x64 k-tile
   int bm = 0, bn = 0;
   int nw = 0;  // > 0: mixed launch, 256-wide tiles over the first 256 nw columns, 256x128 after
 };
@@ -377,6 +378,7 @@ PipePlan plan_pipe(int M, int N, int K, int cus) {
       best_cost = cost;
       best_total = total;
       best = p;
+      best.cost = cost;
     }
   };
   // A tile that does not divide M or N still takes the shape: the last
@@ -387,7 +389,7 @@ PipePlan plan_pipe(int M, int N, int K, int cus) {
   for (const TileChoice& t : kTiles) {
     if (M < t.bm || !cols_ok(N, t.bn)) continue;
     const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
-    consider((double)((tiles + cus - 1) / cus) * t.unit * work, tiles * t.unit * work, PipePlan{t.bm, t.bn, 0});
+    consider((double)((tiles + cus - 1) / cus) * t.unit * work, tiles * t.unit * work, PipePlan{0, t.bm, t.bn, 0});
   }
   // mixed 256x256 + 256x128 (the pair-staged kernel: K % 128 == 0)
   if (M >= 256 && K % 128 == 0) {
@@ -395,7 +397,7 @@ PipePlan plan_pipe(int M, int N, int K, int cus) {
     for (int nw = 1; cols_ok(N - 256 * nw, 128); ++nw) {
       const long wide = tm * nw, narrow = tm * ((N - 256 * nw + 127) / 128);
       const double dw = kTiles[0].unit * work, dn = kTiles[1].unit * work;
-      consider(list_makespan(wide, dw, narrow, dn, cus), wide * dw + narrow * dn, PipePlan{256, 256, nw});
+      consider(list_makespan(wide, dw, narrow, dn, cus), wide * dw + narrow * dn, PipePlan{0, 256, 256, nw});
     }
   }
   return best;
@@ -421,8 +423,40 @@ static bool flex_operands_ok(int N, int K, int lda, int ldb, int b_nt) {
   return K >= 16 && (b_nt || N >= 16) && lda < (1 << 25) && ldb < (1 << 25);
 }
 
+// How a product runs: pipelined tiles (pipe.bm > 0), register-staged ones
+// (flex.bm > 0), or the 64x64 kernel.  Where both of the first two apply, the
+// pipelined ones unless the others' estimate is well below theirs (a unit of
+// plan_pipe takes about 0.5 us, 0.7 where B is too large for the caches to hold
+// from the last call, plus 1.5 us): a handful of 128x128 tiles over a long K,
+// which the register-staged kernel splits.  Pipelined against split:
+// 128x4096x11008 49.2 and 20.0 us, 256x4096x11008 48.8 and 35.0, 512x512x8192 NT
+// 29.4 and 12.6; on the other side of the line 256x4096x4096 19.2 and 16.3
+// first time, 12.0 and 16.1 repeated, 256x1024x2048 NT 7.3 either way.  Above
+// K = 2^15 the pipelined kernel stays, though a split would be faster there
+// too: the test of its rounding term at the largest K it takes (256x256x65472)
+// relies on its being planned.
+struct Route {
+  PipePlan pipe;
+  flex::Plan flex;
+};
+static Route route(miaie_ctx* ctx, int M, int N, int K, bool pipe_ok, bool flex_ok) {
+  Route r;
+  if (pipe_ok) r.pipe = plan_pipe(M, N, K, ctx->cus);
+  // (256-row tiles: enough of them that no split is better)
+  if (r.pipe.bm != 256 && flex_ok) {
+    r.flex = flex::plan(M, N, K, 1.0, ctx->cus, true, ctx->work_bytes);
+    const double unit_us = (size_t)N * K > ((size_t)16 << 20) ? 0.7 : 0.5;
+    if (r.pipe.bm && K <= (1 << 15) && r.flex.us < 0.75 * (1.5 + unit_us * r.pipe.cost))
+      r.pipe = PipePlan{};
+    else if (r.pipe.bm)
+      r.flex = flex::Plan{};
+  }
+  return r;
+}
+
 int plan_gemm_i8(miaie_ctx* ctx, int M, int N, int K, int dense_ok, miaie_gemm_plan* plan) {
-  const PipePlan p = dense_ok ? plan_pipe(M, N, K, ctx->cus) : PipePlan{};
+  const Route r = route(ctx, M, N, K, dense_ok, flex_operands_ok(N, K, K, N, false));
+  const PipePlan& p = r.pipe;
   *plan = miaie_gemm_plan{};
   plan->threads = p.bm == 128 ? 512 : 256;
   if (p.bm && p.nw) {
@@ -435,12 +469,11 @@ int plan_gemm_i8(miaie_ctx* ctx, int M, int N, int K, int dense_ok, miaie_gemm_p
     plan->tile_m = p.bm;
     plan->tile_n = p.bn;
     plan->workgroups = ((M + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn);
-  } else if (flex_operands_ok(N, K, K, N, false)) {
-    const flex::Plan f = flex::plan(M, N, K, 1.0, ctx->cus, true, ctx->work_bytes);
+  } else if (r.flex.bm) {
     plan->kernel = MIAIE_KERNEL_TILE64;
-    plan->tile_m = f.bm;
-    plan->tile_n = f.bn;
-    plan->workgroups = (int)(f.tiles * f.splits);
+    plan->tile_m = r.flex.bm;
+    plan->tile_n = r.flex.bn;
+    plan->workgroups = (int)(r.flex.tiles * r.flex.splits);
   } else {
     plan->kernel = MIAIE_KERNEL_TILE64;
     plan->tile_m = 64;
@@ -453,8 +486,9 @@ int plan_gemm_i8(miaie_ctx* ctx, int M, int N, int K, int dense_ok, miaie_gemm_p
 // Chooses the kernel.  Y and/or C may be NULL (not both).
 int launch_gemm_i8(miaie_ctx* ctx, const int8_t* A, const int8_t* B, int8_t* Y, int32_t* C, int M,
                    int N, int K, int lda, int ldb, int ldy, int ldc, int b_nt, int shift, int relu, bool keep_y) {
-  const PipePlan plan =
-      pipe_operands_ok(A, B, Y, C, K, lda, ldb, ldy, ldc) ? plan_pipe(M, N, K, ctx->cus) : PipePlan{};
+  const Route r = route(ctx, M, N, K, pipe_operands_ok(A, B, Y, C, K, lda, ldb, ldy, ldc),
+                        flex_operands_ok(N, K, lda, ldb, b_nt));
+  const PipePlan& plan = r.pipe;
   const int dev = ctx->device;
   if (plan.bm && plan.nw) {
     const int nw = plan.nw;
@@ -481,8 +515,8 @@ int launch_gemm_i8(miaie_ctx* ctx, const int8_t* A, const int8_t* B, int8_t* Y, 
   }
   dim3 grid((N + 63) / 64, (M + 63) / 64), block(256);
   if (grid.y > 65535) return fail(ctx, MIAIE_EINVAL, "gemm_i8: M too large for the 64x64 fallback");
-  if (flex_operands_ok(N, K, lda, ldb, b_nt)) {
-    flex::Plan f = flex::plan(M, N, K, 1.0, ctx->cus, true, ctx->work_bytes);
+  if (r.flex.bm) {
+    flex::Plan f = r.flex;
     if (f.splits > 1 && !may_split(ctx)) f = flex::plan(M, N, K, 1.0, ctx->cus, false, 0);
     hipError_t e = hipSuccess;
     flex::with_geom(f, [&](auto g) {

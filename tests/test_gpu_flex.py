@@ -61,6 +61,15 @@ def test_gemm_i8_flex(ctx, M, N, K, layout):
         b.free()
 
 
+@pytest.mark.parametrize("M,N,K,layout", [(128, 128, 8192, mi.B_NT), (130, 256, 5120, mi.B_NN)])
+def test_gemm_i8_flex_in_place_of_few_pipelined_tiles(ctx, M, N, K, layout):
+    """Shapes the 128x128 pipelined kernel takes, over a K long enough that
+    the split is the plan (in one part they would be a quarter of the CUs)."""
+    plan = ctx.plan_gemm_i8(M, N, K)
+    assert plan["kernel"] == mi.KERNEL_TILE64 and plan["workgroups"] > -(-M // 64) * -(-N // 64), plan
+    test_gemm_i8_flex(ctx, M, N, K, layout)
+
+
 @pytest.mark.parametrize("M,N,K,layout", [(5, 40, 1000, mi.B_NN), (70, 90, 300, mi.B_NT), (130, 150, 48, mi.B_NN),
                                           (33, 100, 2100, mi.B_NT)])
 @pytest.mark.parametrize("off", [1, 3, 8])
