@@ -460,6 +460,7 @@ struct PixelLoader {
   const RunShape& k;
   int last;        // last offset a 16-byte load may start at
   int r0, ch;
+  int n0, ho0, wo0;  // the thread's first pixel
   int hi0[NL];     // first input row under the filter (negative in the padding)
   int xb[NL];      // first byte of the run within its row (likewise)
   int at0[NL];     // its offset in X
@@ -469,18 +470,35 @@ struct PixelLoader {
   bool edge, shift;
   __device__ __forceinline__ PixelLoader(const int8_t* X_, const RunShape& k_, int total, int p0, int P, int tid)
       : X(X_), k(k_), last(total - 16), r0(tid / G::CH), ch(tid % G::CH), edge(false), shift(false) {
-    // one pixel divided out, the thread's others from there (RPP i further,
-    // at most BM rows and columns: small quotients)
     const uint32_t p = (uint32_t)min(p0 + r0, P - 1), t = p / (uint32_t)k.Wo;
-    const int wo0 = (int)(p - t * k.Wo), n0 = (int)(t / (uint32_t)k.Ho), ho0 = (int)t - n0 * k.Ho;
+    wo0 = (int)(p - t * k.Wo);
+    n0 = (int)(t / (uint32_t)k.Ho);
+    ho0 = (int)t - n0 * k.Ho;
+    rows();
+  }
+  // the tile dn images, dh rows and dw columns further (dh < Ho, dw < Wo)
+  __device__ __forceinline__ void advance(int dn, int dh, int dw) {
+    wo0 += dw;
+    const int cw = wo0 >= k.Wo ? 1 : 0;
+    wo0 -= cw ? k.Wo : 0;
+    ho0 += dh + cw;
+    const int chh = ho0 >= k.Ho ? 1 : 0;
+    ho0 -= chh ? k.Ho : 0;
+    n0 += dn + chh;
+    rows();
+  }
+  // The thread's pixels from its first one: RPP i further, at most BM rows and
+  // columns (small quotients).  Pixels past the last give offsets past the last
+  // image, which load moves inside X: they are never stored.
+  __device__ __forceinline__ void rows() {
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
-      const int x = wo0 + min(G::RPP * i, P - 1 - (int)p);  // (pixels past the last repeat it)
+      const int x = wo0 + G::RPP * i;
       const int dh = k.Wo > G::BM ? (int)(x >= k.Wo) : div_small(x, k.Wo, k.wo_inv);
       const int y = ho0 + dh, dn = k.Ho > G::BM ? (int)(y >= k.Ho) : div_small(y, k.Ho, k.ho_inv);
       hi0[i] = (y - dn * k.Ho) * k.stride - k.pad;
       xb[i] = ((x - dh * k.Wo) * k.stride - k.pad) * k.Cin;
-      at0[i] = ((n0 + dn) * k.H + hi0[i]) * (k.Wd * k.Cin) + xb[i];
+      at0[i] = (int)((uint32_t)((n0 + dn) * k.H + hi0[i]) * (uint32_t)(k.Wd * k.Cin) + (uint32_t)xb[i]);
     }
   }
   __device__ __forceinline__ void load(int s) {
@@ -493,11 +511,11 @@ struct PixelLoader {
     for (int i = 0; i < NL; ++i) {
       // (a row outside the image is loaded from wherever the offset points,
       // moved inside X, and zeroed)
-      const int at = at0[i] + step, from = min(max(at, 0), last), b = xb[i] + 16 * c;
+      const int at = (int)((uint32_t)at0[i] + (uint32_t)step), from = min(max(at, 0), last), b = xb[i] + 16 * c;
       v[i] = MIAIE_LD(reinterpret_cast<const flex::Any16*>(X + (uint32_t)from)).v;
       const int lo = min(max(-b, 0), 16);
       const int up = (unsigned)(hi0[i] + r) < (unsigned)k.H ? min(max(row_bytes - b, 0), 16) : 0;
-      moved[i] = at - from;
+      moved[i] = (int)((uint32_t)at - (uint32_t)from);
       keep[i] = lo | up << 8;
       e |= keep[i] != (16 << 8);
       m |= moved[i] != 0;
@@ -563,11 +581,9 @@ struct WeightLoader {
   }
 };
 
-// Bound by its vector instructions: with few channels a workgroup has one
-// stage, and the pixels' addresses, masks and the requantize outweigh the
-// MFMAs.  8x224x224x3 -> 64, 7x7, stride 2 (1568 tiles of 64x64, one stage of
-// 224 bytes): 12.8 us, 919 with one thread per output; 8x48x48x96 -> 146, 5x5:
-// 29 us.
+// Bound by its vector instructions: the pixels' addresses, masks and the
+// requantize outweigh the MFMAs.  8x48x48x96 -> 146, 5x5 (10 stages): 29 us,
+// 19.9 ms with one thread per output.
 template <class G>
 __global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void conv2d_i8_flex(const int8_t* __restrict__ X, const int8_t* __restrict__ W,
                                                          const uint8_t* __restrict__ shifts, int8_t* __restrict__ Y,
@@ -622,6 +638,93 @@ __global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void conv2d_i8_flex(const
   }
   __syncthreads();
   flex::store_y<G>(lds, Y, Cout, p0, co0, P, Cout, tid);
+}
+
+// The same for a k of one stage and more pixel tiles than workgroups that fit
+// the GPU at once (a network's first layers): a workgroup keeps one channel
+// tile, its weights in LDS and its shifts in registers, and walks over the
+// pixel tiles first, first + step, ..., the next tile's loads in flight while
+// this one is multiplied and stored.  grid.x: TN * step workgroups.
+// 8x224x224x3 -> 64, 7x7, stride 2 (1568 tiles, k of 224 bytes): 11.3 us, 13.2 with
+// a workgroup per tile, 919 with one thread per output; 16x224x224x1 -> 128, 3x3:
+// 43.6 and 70.4 us; 8x201x201x96 -> 128, 1x1, stride 2: 9.2 and 11.8.
+template <class G>
+struct WalkGeom {
+  static constexpr int LDS = G::A_BYTES + G::B_BYTES + G::BM * G::YP;
+};
+template <class G>
+__global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void conv2d_i8_flex_walk(
+    const int8_t* __restrict__ X, const int8_t* __restrict__ W, const uint8_t* __restrict__ shifts,
+    int8_t* __restrict__ Y, RunShape k, int x_bytes, int P, int Cout, int step, int dn, int dh, int dw) {
+  __shared__ __attribute__((aligned(1024))) int8_t lds[WalkGeom<G>::LDS];
+  int8_t* const bs = lds + G::A_BYTES;
+  int8_t* const ys = bs + G::B_BYTES;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / G::WAVES_N, wn = wave % G::WAVES_N;
+  const int TM = (P + G::BM - 1) / G::BM;
+  const int tn = blockIdx.x / step, co0 = tn * G::BN;
+  int tm = blockIdx.x - tn * step;
+  const int fr = lane & 15, fg = lane >> 4;
+
+  PixelLoader<G, G::NA> la(X, k, x_bytes, tm * G::BM, P, tid);
+  WeightLoader<G, G::NB> lb(W, k, co0, Cout, tid);
+  la.load(0);
+  lb.load(0);
+  int sh[G::NJ][4];
+#pragma unroll
+  for (int j = 0; j < G::NJ; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      sh[j][e] = MIAIE_LD(shifts + min(co0 + wn * G::WN + 16 * j + 4 * fg + e, Cout - 1));
+  lb.put(0, bs);
+  const int ksteps = (k.R * k.CPR + 3) / 4;  // 64-byte steps that hold any of k
+
+  while (true) {
+    la.put(0, lds);
+    __syncthreads();  // (and the last tile's output rows have been read)
+    const int next = tm + step;
+    if (next < TM) {
+      la.advance(dn, dh, dw);
+      la.load(0);
+    }
+    v4i acc[G::NI][G::NJ];
+#pragma unroll
+    for (int i = 0; i < G::NI; ++i)
+#pragma unroll
+      for (int j = 0; j < G::NJ; ++j) acc[i][j] = v4i{0};
+#pragma unroll
+    for (int ks = 0; ks < G::KB / 64; ++ks) {
+      if (ks >= ksteps) break;
+      v4i a[G::NI], b[G::NJ];
+#pragma unroll
+      for (int i = 0; i < G::NI; ++i)
+        a[i] = *reinterpret_cast<const v4i*>(lds + flex::row_off(G::KB, wm * G::WM + 16 * i + fr, 4 * ks + fg));
+#pragma unroll
+      for (int j = 0; j < G::NJ; ++j)
+        b[j] = *reinterpret_cast<const v4i*>(bs + flex::row_off(G::KB, wn * G::WN + 16 * j + fr, 4 * ks + fg));
+#pragma unroll
+      for (int i = 0; i < G::NI; ++i)
+#pragma unroll
+        for (int j = 0; j < G::NJ; ++j) acc[i][j] = flex::Mma<int8_t>::mma(b[j], a[i], acc[i][j]);
+    }
+    // (k of one stage: |acc| < 2^22, room for the rounding term)
+#pragma unroll
+    for (int j = 0; j < G::NJ; ++j) {
+      const int nl = wn * G::WN + 16 * j + 4 * fg;
+#pragma unroll
+      for (int i = 0; i < G::NI; ++i) {
+        uint32_t y = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          y |= (uint32_t)(min(max((acc[i][j][e] + (int)((1u << sh[j][e]) >> 1)) >> sh[j][e], -128), 127) & 0xFF) << (8 * e);
+        *reinterpret_cast<uint32_t*>(ys + (wm * G::WM + 16 * i + fr) * G::YP + nl) = y;
+      }
+    }
+    __syncthreads();  // the output rows are whole, the pixels' LDS is free
+    flex::store_y<G>(ys, Y, Cout, tm * G::BM, co0, P, Cout, tid);
+    if (next >= TM) break;
+    tm = next;
+  }
 }
 
 // Operands of fewer than 16 bytes, and above 2^31: one thread per output
@@ -823,6 +926,19 @@ static int launch_flex(miaie_ctx* ctx, const int8_t* X, const int8_t* W, const u
   hipError_t e = hipSuccess;
   flex::with_geom(f, [&](auto g) {
     using G = typename decltype(g)::type;
+    const long tn = (Cout + G::BN - 1) / G::BN, tm = f.tiles / tn;
+    // one stage, and pixel tiles for more than one round of the workgroups
+    // that fit (by LDS and registers, 4 per CU, 2 of 128x128).  (Fewer
+    // workgroups, each with the same number of tiles: 12.7 us against 11.3 for
+    // 8x224x224x3 -> 64, 7x7, stride 2.)
+    const long step = std::max(1l, (G::BM < 128 ? 4l : 2l) * ctx->cus / tn);
+    if (16 * R * k.CPR <= G::KB && tm > step) {
+      const long pixels = step * G::BM;  // from one of a workgroup's tiles to its next
+      e = launch<conv2d_i8_flex_walk<G>>(ctx->device, dim3((unsigned)(tn * step)), dim3(256), 0, ctx->stream, X, W,
+                                         shifts, Y, k, N * H * Wd * Cin, (int)P, Cout, (int)step,
+                                         (int)(pixels / Wo / Ho), (int)(pixels / Wo % Ho), (int)(pixels % Wo));
+      return;
+    }
     e = launch<conv2d_i8_flex<G>>(ctx->device, dim3((unsigned)f.tiles, (unsigned)f.splits), dim3(256), 0, ctx->stream, X,
                                   W, shifts, Y, k, N * H * Wd * Cin, (int)P, Cout, static_cast<int8_t*>(ctx->work),
                                   ctx->counters);

@@ -231,6 +231,10 @@ CONV_SHAPES = [
     (1, 3, 3, 7300, 5, 3, 3, 1, 1),   # k >= 2^16: the requant form without the rounding add
     (4, 64, 64, 3, 130, 3, 3, 1, 1),  # 256 x 2 tiles: 128 x 128
     (8, 96, 96, 32, 192, 1, 1, 1, 0),  # a large grid of the implicit-GEMM shapes
+    # one stage of k and more pixel tiles than fit at once: walked over
+    (1, 260, 262, 3, 20, 3, 3, 1, 1),   # rows longer than a tile
+    (2100, 6, 7, 3, 10, 3, 3, 1, 1),    # images smaller than a tile
+    (70000, 2, 1, 16, 70, 1, 1, 1, 0),  # one column, two channel tiles, the last partial
 ]
 
 
