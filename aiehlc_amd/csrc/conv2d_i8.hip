@@ -588,7 +588,7 @@ template <class G>
 __global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void conv2d_i8_flex(const int8_t* __restrict__ X, const int8_t* __restrict__ W,
                                                          const uint8_t* __restrict__ shifts, int8_t* __restrict__ Y,
                                                          RunShape k, int x_bytes, int P, int Cout,
-                                                         int8_t* __restrict__ work, uint32_t* __restrict__ counters) {
+                                                         int8_t* __restrict__ work, int splits) {
   __shared__ __attribute__((aligned(1024))) int8_t lds[G::LDS];
   __shared__ int flag;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -596,7 +596,7 @@ __global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void conv2d_i8_flex(const
   int tm, tn;
   miaie::dev::tile_coords<4>(blockIdx.x, (P + G::BM - 1) / G::BM, (Cout + G::BN - 1) / G::BN, tm, tn);
   const int p0 = tm * G::BM, co0 = tn * G::BN;
-  const int stages = (k.R * k.CPR + G::CH - 1) / G::CH, splits = gridDim.y, split = blockIdx.y;
+  const int stages = (k.R * k.CPR + G::CH - 1) / G::CH, split = blockIdx.y;
   const int s0 = (int)((long long)stages * split / splits), s1 = (int)((long long)stages * (split + 1) / splits);
 
   v4i acc[G::NI][G::NJ];
@@ -616,7 +616,7 @@ __global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void conv2d_i8_flex(const
   WeightLoader<G, G::NB> lb(W, k, co0, Cout, tid);
   flex::tile_loop<int8_t, G, false>(lds, la, lb, s0, s1, lane, wm, wn, acc);
   if (splits > 1 &&
-      !flex::split_sum<int8_t, G>(acc, blockIdx.x, split, splits, work, counters, &flag, tid))
+      !flex::split_sum<int8_t, G>(acc, blockIdx.x, split, splits, work, miaie::ctx_counters(work), &flag, tid))
     return;
 
 #pragma unroll
@@ -940,8 +940,7 @@ static int launch_flex(miaie_ctx* ctx, const int8_t* X, const int8_t* W, const u
       return;
     }
     e = launch<conv2d_i8_flex<G>>(ctx->device, dim3((unsigned)f.tiles, (unsigned)f.splits), dim3(256), 0, ctx->stream, X,
-                                  W, shifts, Y, k, N * H * Wd * Cin, (int)P, Cout, static_cast<int8_t*>(ctx->work),
-                                  ctx->counters);
+                                  W, shifts, Y, k, N * H * Wd * Cin, (int)P, Cout, static_cast<int8_t*>(ctx->work), f.splits);
   });
   return check_launch(ctx, e, "conv2d_i8_flex");
 }

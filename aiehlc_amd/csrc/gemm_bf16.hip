@@ -625,8 +625,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_tile64(const uint16_t* __restri
 template <class G>
 __global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void gemm_bf16_flex(const uint16_t* __restrict__ A,
                                                          const uint16_t* __restrict__ B, float* __restrict__ C,
-                                                         int M, int N, int K, int8_t* __restrict__ work,
-                                                         uint32_t* __restrict__ counters) {
+                                                         int M, int N, int K, int8_t* __restrict__ work, int splits) {
   __shared__ __attribute__((aligned(1024))) int8_t lds[G::LDS];
   __shared__ int flag;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -634,7 +633,7 @@ __global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void gemm_bf16_flex(const
   int tm, tn;
   dev::tile_coords<4>(blockIdx.x, (M + G::BM - 1) / G::BM, (N + G::BN - 1) / G::BN, tm, tn);
   const int m0 = tm * G::BM, n0 = tn * G::BN;
-  const int stages = (2 * K + G::KB - 1) / G::KB, splits = gridDim.y, split = blockIdx.y;
+  const int stages = (2 * K + G::KB - 1) / G::KB, split = blockIdx.y;
   const int s0 = (int)((long long)stages * split / splits), s1 = (int)((long long)stages * (split + 1) / splits);
 
   v4f acc[G::NI][G::NJ];
@@ -646,7 +645,7 @@ __global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void gemm_bf16_flex(const
   flex::ColsLoader<uint16_t, G, true> lb(reinterpret_cast<const int8_t*>(B), n0, N, (size_t)N * 2, K, tid);
   flex::tile_loop<uint16_t, G, true>(lds, la, lb, s0, s1, lane, wm, wn, acc);
   if (splits > 1 &&
-      !flex::split_sum<uint16_t, G>(acc, blockIdx.x, split, splits, work, counters, &flag, tid))
+      !flex::split_sum<uint16_t, G>(acc, blockIdx.x, split, splits, work, miaie::ctx_counters(work), &flag, tid))
     return;
 
   const int fr = lane & 15, fg = lane >> 4;
@@ -693,7 +692,7 @@ int launch_gemm_bf16(miaie_ctx* ctx, const uint16_t* A, const uint16_t* B, float
     flex::with_geom(f, [&](auto g) {
       using G = typename decltype(g)::type;
       e = launch<gemm_bf16_flex<G>>(ctx->device, dim3((unsigned)f.tiles, (unsigned)f.splits), dim3(256), 0, ctx->stream,
-                                    A, B, C, M, N, K, static_cast<int8_t*>(ctx->work), ctx->counters);
+                                    A, B, C, M, N, K, static_cast<int8_t*>(ctx->work), f.splits);
     });
     return check_launch(ctx, e, "gemm_bf16_flex");
   }

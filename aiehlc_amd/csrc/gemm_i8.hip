@@ -138,7 +138,8 @@ __global__ __launch_bounds__(256) void gemm_i8_tile64(const int8_t* __restrict__
 
 // Register-staged tiles (flex_tile.hpp): any size, stride and alignment with
 // rows of at least 16 bytes.  grid.x: output tiles, grid.y: the `splits`
-// workgroups that divide a tile's K.  Bound by the latency of the stages'
+// workgroups that divide a tile's K; mode: shift, relu << 8, splits << 16 (one
+// argument: each costs the launch host time).  Bound by the latency of the stages'
 // loads, and for few rows by reading B: 1000 x 2050 x 1000 NT (rows of 1000
 // bytes) took 61.1 us in the byte-wise 64x64 kernel and takes 8.8; the MLP
 // over 16 rows (4096 -> 11008 -> 4096, 90 MB of weights) 204.7 us in a
@@ -147,8 +148,9 @@ __global__ __launch_bounds__(256) void gemm_i8_tile64(const int8_t* __restrict__
 template <class G, bool B_NT>
 __global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void gemm_i8_flex(const int8_t* __restrict__ A, const int8_t* __restrict__ B,
                                                        int8_t* __restrict__ Y, int32_t* __restrict__ C, int M, int N,
-                                                       int K, int lda, int ldb, int ldy, int ldc, int shift, int relu,
-                                                       int8_t* __restrict__ work, uint32_t* __restrict__ counters) {
+                                                       int K, int lda, int ldb, int ldy, int ldc, uint32_t mode,
+                                                       int8_t* __restrict__ work) {
+  const int shift = mode & 31, relu = (mode >> 8) & 1, splits = mode >> 16;
   __shared__ __attribute__((aligned(1024))) int8_t lds[G::LDS];
   __shared__ int flag;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -156,7 +158,7 @@ __global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void gemm_i8_flex(const i
   int tm, tn;
   flex::tile_index<!B_NT && G::BN == 64>((M + G::BM - 1) / G::BM, (N + G::BN - 1) / G::BN, tm, tn);
   const int m0 = tm * G::BM, n0 = tn * G::BN;
-  const int stages = (K + G::KB - 1) / G::KB, splits = gridDim.y, split = blockIdx.y;
+  const int stages = (K + G::KB - 1) / G::KB, split = blockIdx.y;
   const int s0 = (int)((long long)stages * split / splits), s1 = (int)((long long)stages * (split + 1) / splits);
 
   v4i acc[G::NI][G::NJ];
@@ -173,7 +175,7 @@ __global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void gemm_i8_flex(const i
     flex::tile_loop<int8_t, G, true>(lds, la, lb, s0, s1, lane, wm, wn, acc);
   }
   if (splits > 1 &&
-      !flex::split_sum<int8_t, G>(acc, blockIdx.x, split, splits, work, counters, &flag, tid))
+      !flex::split_sum<int8_t, G>(acc, blockIdx.x, split, splits, work, miaie::ctx_counters(work), &flag, tid))
     return;
 
   const int fr = lane & 15, fg = lane >> 4, lo = relu ? 0 : -128;
@@ -523,10 +525,11 @@ int launch_gemm_i8(miaie_ctx* ctx, const int8_t* A, const int8_t* B, int8_t* Y, 
       using G = typename decltype(g)::type;
       const dim3 fg((unsigned)f.tiles, (unsigned)f.splits);
       int8_t* const work = static_cast<int8_t*>(ctx->work);
+      const uint32_t mode = (uint32_t)(shift | relu << 8 | f.splits << 16);
       e = b_nt ? launch<gemm_i8_flex<G, true>>(dev, fg, block, 0, ctx->stream, A, B, Y, C, M, N, K, lda, ldb, ldy, ldc,
-                                               shift, relu, work, ctx->counters)
+                                               mode, work)
                : launch<gemm_i8_flex<G, false>>(dev, fg, block, 0, ctx->stream, A, B, Y, C, M, N, K, lda, ldb, ldy, ldc,
-                                                shift, relu, work, ctx->counters);
+                                                mode, work);
     });
     return check_launch(ctx, e, "gemm_i8_flex");
   }

@@ -24,11 +24,11 @@ struct miaie_ctx {
   void* scratch = nullptr;    // device address of this device's file-scope scratch array (noalloc.hip)
   // Device workspace owned by this context, allocated once at init so that
   // no entry point allocates: split-K partial sums, and the arrival counters
-  // of the tiles whose K is split (flex::split_sum; every launch leaves them
-  // at 0).  Work queued on the context's one stream uses it in stream order.
+  // of the tiles whose K is split (MIAIE_CTX_COUNTERS of them at
+  // ctx_counters(work); flex::split_sum: every launch leaves them at 0).
+  // Work queued on the context's one stream uses it in stream order.
   void* work = nullptr;
   size_t work_bytes = 0;
-  uint32_t* counters = nullptr;  // MIAIE_CTX_COUNTERS of them, behind the work_bytes
   char err[512] = {0};
 };
 
@@ -36,6 +36,11 @@ constexpr size_t MIAIE_CTX_WORK_BYTES = (size_t)16 << 20;
 constexpr int MIAIE_CTX_COUNTERS = 4096;
 
 namespace miaie {
+
+// The arrival counters behind a context's workspace.
+__host__ __device__ inline uint32_t* ctx_counters(void* work) {
+  return reinterpret_cast<uint32_t*>(static_cast<int8_t*>(work) + MIAIE_CTX_WORK_BYTES);
+}
 
 // Record an error message on the context (printf-style) and return `code`.
 int fail(miaie_ctx* ctx, int code, const char* fmt, ...) __attribute__((format(printf, 3, 4)));

@@ -266,8 +266,7 @@ extern "C" int miaie_init_on_stream(miaie_ctx** out, int device, void* stream) {
   e = hipMalloc(&ctx->work, MIAIE_CTX_WORK_BYTES + kCounterBytes);
   if (e == hipSuccess) {
     ctx->work_bytes = MIAIE_CTX_WORK_BYTES;
-    ctx->counters = reinterpret_cast<uint32_t*>(static_cast<int8_t*>(ctx->work) + MIAIE_CTX_WORK_BYTES);
-    e = hipMemset(ctx->counters, 0, kCounterBytes);
+    e = hipMemset(ctx_counters(ctx->work), 0, kCounterBytes);
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);  // done before any stream uses them
   }
   if (e != hipSuccess) {
