@@ -268,7 +268,7 @@ MIAIE_API int miaie_gemm_bf16_f32(miaie_ctx* ctx, const uint16_t* A, const uint1
  * Cin a multiple of 128 with Cout a multiple of 64 the LDS-staged taps
  * kernel; Cin a multiple of 32 with Cout a multiple of 64 the implicit-GEMM
  * kernel (the last two split K over workgroups for small grids, through the
- * context's workspace); everything else a direct kernel
+ * context's workspace); everything else the register-staged kernel
  * (miaie_plan_conv2d_i8 reports which).
  * R*S*Cin above 2^30 or N*H*W*Cin above 2^40 return MIAIE_EINVAL. */
 MIAIE_API int miaie_conv2d_i8_nhwc(miaie_ctx* ctx, const int8_t* X, const int8_t* W,
