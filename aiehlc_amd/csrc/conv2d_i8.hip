@@ -840,20 +840,32 @@ static double rows128_us(int N, int Ho, int Wo, int Cout, int cus) {
 
 // conv2d_i8_taps as its launcher runs it: 128 x 128 tiles when they fill a
 // round of CUs, else 64 x 64 split over k; a stage is one tap x 128 channels.
+static bool taps_big(size_t P, int Cout, int cus) {
+  return Cout % 128 == 0 && ((P + 127) / 128) * (size_t)(Cout / 128) >= (size_t)cus;
+}
+static int taps_ksplit(size_t P, int Cin, int Cout, int R, int S, int cus, size_t work_bytes) {
+  if (taps_big(P, Cout, cus)) return 1;
+  return conv_ksplit(((P + 63) / 64) * (size_t)(Cout / 64), R * S * (Cin / 128), 4, P * Cout, cus, work_bytes);
+}
 static double taps_us(size_t P, int Cin, int Cout, int R, int S, int cus, size_t work_bytes) {
   const int stages = R * S * (Cin / 128);
   const size_t t128 = ((P + 127) / 128) * (size_t)(Cout / 128);
-  if (Cout % 128 == 0 && t128 >= (size_t)cus) return launch_rounds(t128, cus) * (4.0 + 0.69 * stages);
+  if (taps_big(P, Cout, cus)) return launch_rounds(t128, cus) * (4.0 + 0.69 * stages);
   const size_t t64 = ((P + 63) / 64) * (size_t)(Cout / 64);
-  const int ks = conv_ksplit(t64, stages, 4, P * Cout, cus, work_bytes);
+  const int ks = taps_ksplit(P, Cin, Cout, R, S, cus, work_bytes);
   return launch_rounds(t64 * ks, cus) * (2.5 + 0.41 * stages / ks) + (ks > 1 ? 3.0 : 0.0);
+}
+
+static int igemm_ksplit(size_t P, int Cin, int Cout, int R, int S, int cus, size_t work_bytes) {
+  return conv_ksplit(((P + PIX - 1) / PIX) * (size_t)(Cout / COB), R * S * (Cin / 32), 4 * BATCH, P * Cout, cus, work_bytes);
 }
 
 // The kernel choice weighs estimated times on `cus` compute units: the
 // context's count at launch (miaie_plan_set_cus or the device's), and an
-// MI355X's 256 for miaie_plan_conv2d_i8, which has no context.
+// MI355X's 256 for miaie_plan_conv2d_i8, which has no context.  work_bytes:
+// room for split-K partial sums (0: no split).
 int conv2d_kernel_for(int N, int H, int Wd, int Cin, int Cout, int R, int S, int stride, int pad, bool aligned16,
-                      bool shifts_aligned4, int cus) {
+                      bool shifts_aligned4, int cus, size_t work_bytes) {
   const int Ho = (H + 2 * pad - R) / stride + 1;
   const int Wo = (Wd + 2 * pad - S) / stride + 1;
   const size_t P = (size_t)N * Ho * Wo;
@@ -890,7 +902,7 @@ int conv2d_kernel_for(int N, int H, int Wd, int Cin, int Cout, int R, int S, int
   if (deep_ok && taps_ok) {
     const RowsDeepTile t = rows_deep_tile(N, Ho, Wo, Cin, Cout, cus);
     return rows_deep_us(N, Ho, Wo, Cin, Cout, t, cus) <=
-                   taps_us(P, Cin, Cout, R, S, cus, MIAIE_CTX_WORK_BYTES)
+                   taps_us(P, Cin, Cout, R, S, cus, work_bytes)
                ? MIAIE_CONV_ROWS_DEEP
                : MIAIE_CONV_TAPS;
   }
@@ -950,9 +962,15 @@ int launch_conv2d_i8(miaie_ctx* ctx, const int8_t* X, const int8_t* W, const uin
   const int Ho = (H + 2 * pad - R) / stride + 1;
   const int Wo = (Wd + 2 * pad - S) / stride + 1;
   const size_t P = (size_t)N * Ho * Wo;
-  const int kernel = conv2d_kernel_for(N, H, Wd, Cin, Cout, R, S, stride, pad,
-                                       aligned(X, 16) && aligned(W, 16) && aligned(Y, 16), aligned(shifts, 4),
-                                       ctx->cus);
+  const bool al16 = aligned(X, 16) && aligned(W, 16) && aligned(Y, 16), al4 = aligned(shifts, 4);
+  int kernel = conv2d_kernel_for(N, H, Wd, Cin, Cout, R, S, stride, pad, al16, al4, ctx->cus, ctx->work_bytes);
+  int ks = kernel == MIAIE_CONV_TAPS    ? taps_ksplit(P, Cin, Cout, R, S, ctx->cus, ctx->work_bytes)
+           : kernel == MIAIE_CONV_IGEMM ? igemm_ksplit(P, Cin, Cout, R, S, ctx->cus, ctx->work_bytes)
+                                        : 1;
+  if (ks > 1 && !may_split(ctx)) {  // planned again without the workspace
+    kernel = conv2d_kernel_for(N, H, Wd, Cin, Cout, R, S, stride, pad, al16, al4, ctx->cus, 0);
+    ks = 1;
+  }
   if (kernel == MIAIE_CONV_ROWS) {
     if (Cin == 128) return launch_rows<128>(ctx, X, W, shifts, Y, N, H, Wd, Cout, pad, Ho, Wo);
     if (Cin == 64) return launch_rows<64>(ctx, X, W, shifts, Y, N, H, Wd, Cout, pad, Ho, Wo);
@@ -975,11 +993,9 @@ int launch_conv2d_i8(miaie_ctx* ctx, const int8_t* X, const int8_t* W, const uin
   if (kernel == MIAIE_CONV_TAPS) {
     // 128 x 128 tiles when they fill at least one round of CUs, else 64 x 64
     // (split over k when even those leave most CUs idle)
-    const bool big = Cout % 128 == 0 && ((P + 127) / 128) * (size_t)(Cout / 128) >= (size_t)ctx->cus;
+    const bool big = taps_big(P, Cout, ctx->cus);
     const int tp = big ? 128 : 64;
     const unsigned pxb = (unsigned)((P + tp - 1) / tp), chb = (unsigned)(Cout / tp);
-    const int ks = big ? 1 : conv_ksplit((size_t)pxb * chb, R * S * (Cin / 128), 4, P * Cout, ctx->cus,
-                                             ctx->work_bytes);
     const int dev = ctx->device;
     if (big) {
       const hipError_t e = launch<conv2d_i8_taps<128, 128, false>>(dev, dim3(pxb, chb, 1), dim3(256), 0, ctx->stream,
@@ -1013,7 +1029,6 @@ int launch_conv2d_i8(miaie_ctx* ctx, const int8_t* X, const int8_t* W, const uin
   const bool flex = flex_ok(N, H, Wd, Cin, Cout, R, S, pad, P);
   if (kernel == MIAIE_CONV_IGEMM && !(big && flex)) {
     const unsigned pxb = (unsigned)((P + PIX - 1) / PIX), chb = (unsigned)(Cout / COB);
-    const int ks = conv_ksplit((size_t)pxb * chb, R * S * (Cin / 32), 4 * BATCH, P * Cout, ctx->cus, ctx->work_bytes);
     if (ks > 1) {
       int32_t* const part = static_cast<int32_t*>(ctx->work);
       hipError_t e = launch<conv2d_i8_igemm<true>>(ctx->device, dim3(pxb, chb, (unsigned)ks), dim3(256), 0,

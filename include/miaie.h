@@ -189,7 +189,9 @@ MIAIE_API int miaie_plan_conv2d_i8(int N, int H, int W, int Cin, int Cout, int R
  * the context that recorded it (another context gets MIAIE_EINVAL), before
  * that context's miaie_finish: a recorded product or convolution may use the
  * context's workspace.  (While the caller captures the context's stream with
- * HIP itself, GEMMs are not split over K and so leave the workspace alone.) */
+ * HIP itself, neither GEMMs nor convolutions are split over K: their graph may
+ * be replayed beside other work of the context, and leaves the workspace
+ * alone.) */
 typedef struct miaie_graph miaie_graph;
 MIAIE_API int miaie_graph_begin(miaie_ctx* ctx);
 MIAIE_API int miaie_graph_end(miaie_ctx* ctx, miaie_graph** graph);

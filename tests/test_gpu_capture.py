@@ -1,0 +1,137 @@
+"""Entry points recorded by the caller's own HIP capture of the context's
+stream (not miaie_graph_begin).  Such a graph may be replayed on any stream,
+beside other work of the context, so what it holds must not touch the
+context's workspace: no split of K."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import aiehlc_amd as mi
+import oracle
+from aiehlc_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+NON_BLOCKING, THREAD_LOCAL = 1, 1  # hipStreamNonBlocking, hipStreamCaptureModeThreadLocal
+
+
+class _Dim3(C.Structure):
+    _fields_ = [("x", C.c_uint), ("y", C.c_uint), ("z", C.c_uint)]
+
+
+class _KernelNodeParams(C.Structure):  # hipKernelNodeParams
+    _fields_ = [("blockDim", _Dim3), ("extra", C.c_void_p), ("func", C.c_void_p), ("gridDim", _Dim3),
+                ("kernelParams", C.c_void_p), ("sharedMemBytes", C.c_uint)]
+
+
+class Capture:
+    """A context on a stream of the caller's, and a second stream for replays."""
+
+    def __init__(self):
+        self.hip = C.CDLL("libamdhip64.so")
+        self.streams = [C.c_void_p(), C.c_void_p()]
+        for s in self.streams:
+            self.ok(self.hip.hipStreamCreateWithFlags(C.byref(s), NON_BLOCKING))
+        self.ctx = mi.Context(0, stream=self.streams[0].value)
+
+    def ok(self, rc):
+        assert rc == 0, rc
+
+    def record(self, call):
+        """(graph executable, grid of each kernel node)"""
+        hip, graph, exe, n = self.hip, C.c_void_p(), C.c_void_p(), C.c_size_t()
+        self.ok(hip.hipStreamBeginCapture(self.streams[0], THREAD_LOCAL))
+        try:
+            call()
+        finally:
+            rc = hip.hipStreamEndCapture(self.streams[0], C.byref(graph))
+        self.ok(rc)
+        self.ok(hip.hipGraphGetNodes(graph, None, C.byref(n)))
+        nodes = (C.c_void_p * n.value)()
+        self.ok(hip.hipGraphGetNodes(graph, nodes, C.byref(n)))
+        grids = []
+        for node in nodes:
+            p = _KernelNodeParams()
+            self.ok(hip.hipGraphKernelNodeGetParams(C.c_void_p(node), C.byref(p)))
+            grids.append((p.gridDim.x, p.gridDim.y, p.gridDim.z))
+        self.ok(hip.hipGraphInstantiate(C.byref(exe), graph, None, None, 0))
+        self.ok(hip.hipGraphDestroy(graph))
+        return exe, grids
+
+    def replay(self, exe):
+        self.ok(self.hip.hipGraphLaunch(exe, self.streams[1]))
+
+    def sync(self):
+        for s in self.streams:
+            self.ok(self.hip.hipStreamSynchronize(s))
+
+    def close(self):
+        self.sync()
+        self.ctx.close()
+        for s in self.streams:
+            self.ok(self.hip.hipStreamDestroy(s))
+
+
+@pytest.fixture(scope="module")
+def cap():
+    c = Capture()
+    yield c
+    c.close()
+
+
+def _beside_eager_splits(cap, exe, fill_out, check_out):
+    """Replays on the second stream while the context runs products that
+    are split over K through its workspace."""
+    ctx = cap.ctx
+    M, N, K = 16, 512, 8192
+    assert ctx.plan_gemm_i8(M, N, K)["workgroups"] > -(-M // 16) * -(-N // 128)  # split
+    A, B = synth.int8((M, K), 1), synth.int8((K, N), 2)
+    dA, dB, dY = ctx.upload(A), ctx.upload(B), ctx.empty((M, N), np.int8)
+    want = oracle.gemm_i8_rq(A, B, 11)
+    for rep in range(4):
+        fill_out()
+        ctx.copy_h2d(dY, np.full((M, N), 77, np.int8))
+        cap.sync()
+        for _ in range(6):
+            cap.replay(exe)
+            ctx.gemm_i8_rq(dA, dB, dY, M, N, K, 11)
+        cap.sync()
+        check_out(rep)
+        assert np.array_equal(ctx.download(dY), want), rep
+    for b in (dA, dB, dY):
+        b.free()
+    cap.ok(cap.hip.hipGraphExecDestroy(exe))
+
+
+CONV_SHAPES = [
+    # N, H, W, Cin, Cout, R, stride, pad
+    (8, 7, 7, 512, 512, 3, 2, 1),    # taps kernel, split when run directly
+    (8, 7, 7, 512, 512, 3, 1, 1),    # taps against the chunked row-block kernel
+    (1, 7, 7, 96, 64, 5, 1, 2),      # implicit GEMM on fragments from memory
+    (1, 13, 13, 130, 70, 5, 1, 2),   # register-staged tiles
+]
+
+
+@pytest.mark.parametrize("shape", CONV_SHAPES)
+def test_captured_conv_leaves_the_workspace_alone(cap, shape):
+    N, H, W, Cin, Cout, R, stride, pad = shape
+    print(f"[case] captured conv {shape}", flush=True)
+    ctx = cap.ctx
+    rng = np.random.default_rng(sum(shape))
+    X, Wt = (rng.integers(-128, 128, size=s, dtype=np.int8) for s in ((N, H, W, Cin), (Cout, R, R, Cin)))
+    sh = rng.integers(8, 13, size=Cout, dtype=np.uint8)
+    want = oracle.conv2d_nhwc_i8(X, Wt, sh, stride, pad)
+    dX, dW, dS, dY = ctx.upload(X), ctx.upload(Wt), ctx.upload(sh), ctx.empty(want.shape, np.int8)
+    exe, grids = cap.record(lambda: ctx.conv2d_i8_nhwc(dX, dW, dS, dY, N, H, W, Cin, Cout, R, R, stride, pad))
+    # one kernel (a split taps or implicit-GEMM launch is followed by its sum),
+    # and one workgroup per 64 x 64 tile at most (splits are in y or z)
+    P = want.size // Cout
+    assert len(grids) == 1 and np.prod(grids[0]) <= -(-P // 16) * -(-Cout // 32), grids
+
+    def check(rep):
+        assert np.array_equal(ctx.download(dY), want), rep
+
+    _beside_eager_splits(cap, exe, lambda: ctx.copy_h2d(dY, np.full(want.shape, 77, np.int8)), check)
+    for b in (dX, dW, dS, dY):
+        b.free()
