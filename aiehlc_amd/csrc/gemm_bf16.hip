@@ -673,7 +673,10 @@ int launch_gemm_bf16(miaie_ctx* ctx, const uint16_t* A, const uint16_t* B, float
   const bool flexible = K >= 8 && N >= 8 && K < (1 << 24) && N < (1 << 24);
   const dim3 grid((N + 63) / 64, (M + 63) / 64);
   flex::Plan f;
-  if (flexible) f = flex::plan(M, N, 2l * K, 1.0, ctx->cus, true, ctx->work_bytes);
+  if (flexible) {
+    f = flex::plan(M, N, 2l * K, 1.0, ctx->cus, true, ctx->work_bytes);
+    if (f.splits > 1 && !may_split(ctx)) f = flex::plan(M, N, 2l * K, 1.0, ctx->cus, false, 0);
+  }
   // Where both apply, the one estimated faster: a round of 256x256 tiles takes
   // about 3 us and 0.0185 us per k (1024^3, 16 tiles: 23.6 us, 8.5 on 256 of
   // 64x64; 2048x4096x2048, 128 tiles: 43.1 us, as on 512 of 128x128).
@@ -687,7 +690,6 @@ int launch_gemm_bf16(miaie_ctx* ctx, const uint16_t* A, const uint16_t* B, float
   }
   if (grid.y > 65535) return fail(ctx, MIAIE_EINVAL, "gemm_bf16: M too large for the 64x64 fallback");
   if (flexible) {
-    if (f.splits > 1 && !may_split(ctx)) f = flex::plan(M, N, 2l * K, 1.0, ctx->cus, false, 0);
     hipError_t e = hipSuccess;
     flex::with_geom(f, [&](auto g) {
       using G = typename decltype(g)::type;

@@ -441,12 +441,12 @@ struct Route {
   PipePlan pipe;
   flex::Plan flex;
 };
-static Route route(miaie_ctx* ctx, int M, int N, int K, bool pipe_ok, bool flex_ok) {
+static Route route(miaie_ctx* ctx, int M, int N, int K, bool pipe_ok, bool flex_ok, bool can_split) {
   Route r;
   if (pipe_ok) r.pipe = plan_pipe(M, N, K, ctx->cus);
   // (256-row tiles: enough of them that no split is better)
   if (r.pipe.bm != 256 && flex_ok) {
-    r.flex = flex::plan(M, N, K, 1.0, ctx->cus, true, ctx->work_bytes);
+    r.flex = flex::plan(M, N, K, 1.0, ctx->cus, can_split, ctx->work_bytes);
     const double unit_us = (size_t)N * K > ((size_t)16 << 20) ? 0.7 : 0.5;
     if (r.pipe.bm && K <= (1 << 15) && r.flex.us < 0.75 * (1.5 + unit_us * r.pipe.cost))
       r.pipe = PipePlan{};
@@ -457,7 +457,7 @@ static Route route(miaie_ctx* ctx, int M, int N, int K, bool pipe_ok, bool flex_
 }
 
 int plan_gemm_i8(miaie_ctx* ctx, int M, int N, int K, int dense_ok, miaie_gemm_plan* plan) {
-  const Route r = route(ctx, M, N, K, dense_ok, flex_operands_ok(N, K, K, N, false));
+  const Route r = route(ctx, M, N, K, dense_ok, flex_operands_ok(N, K, K, N, false), true);
   const PipePlan& p = r.pipe;
   *plan = miaie_gemm_plan{};
   plan->threads = p.bm == 128 ? 512 : 256;
@@ -488,8 +488,9 @@ int plan_gemm_i8(miaie_ctx* ctx, int M, int N, int K, int dense_ok, miaie_gemm_p
 // Chooses the kernel.  Y and/or C may be NULL (not both).
 int launch_gemm_i8(miaie_ctx* ctx, const int8_t* A, const int8_t* B, int8_t* Y, int32_t* C, int M,
                    int N, int K, int lda, int ldb, int ldy, int ldc, int b_nt, int shift, int relu, bool keep_y) {
-  const Route r = route(ctx, M, N, K, pipe_operands_ok(A, B, Y, C, K, lda, ldb, ldy, ldc),
-                        flex_operands_ok(N, K, lda, ldb, b_nt));
+  const bool pipe_ok = pipe_operands_ok(A, B, Y, C, K, lda, ldb, ldy, ldc), flex_ok = flex_operands_ok(N, K, lda, ldb, b_nt);
+  Route r = route(ctx, M, N, K, pipe_ok, flex_ok, true);
+  if (r.flex.splits > 1 && !may_split(ctx)) r = route(ctx, M, N, K, pipe_ok, flex_ok, false);
   const PipePlan& plan = r.pipe;
   const int dev = ctx->device;
   if (plan.bm && plan.nw) {
@@ -518,8 +519,7 @@ int launch_gemm_i8(miaie_ctx* ctx, const int8_t* A, const int8_t* B, int8_t* Y, 
   dim3 grid((N + 63) / 64, (M + 63) / 64), block(256);
   if (grid.y > 65535) return fail(ctx, MIAIE_EINVAL, "gemm_i8: M too large for the 64x64 fallback");
   if (r.flex.bm) {
-    flex::Plan f = r.flex;
-    if (f.splits > 1 && !may_split(ctx)) f = flex::plan(M, N, K, 1.0, ctx->cus, false, 0);
+    const flex::Plan& f = r.flex;
     hipError_t e = hipSuccess;
     flex::with_geom(f, [&](auto g) {
       using G = typename decltype(g)::type;

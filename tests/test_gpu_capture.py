@@ -135,3 +135,52 @@ def test_captured_conv_leaves_the_workspace_alone(cap, shape):
     _beside_eager_splits(cap, exe, lambda: ctx.copy_h2d(dY, np.full(want.shape, 77, np.int8)), check)
     for b in (dX, dW, dS, dY):
         b.free()
+
+
+GEMM_SHAPES = [
+    # M, N, K, workgroups of the plan without a split, at 256 CUs
+    (16, 512, 8192, 8),              # register-staged 64 x 64
+    (512, 512, 8192, 16),            # the pipelined 128 x 128 kernel: faster than register-staged tiles unsplit
+    (130, 300, 2049, 15),            # register-staged, ragged
+]
+
+
+@pytest.mark.parametrize("M,N,K,workgroups", GEMM_SHAPES)
+@pytest.mark.parametrize("layout", [mi.B_NN, mi.B_NT])
+def test_captured_int8_gemm_is_planned_without_a_split(cap, M, N, K, workgroups, layout):
+    print(f"[case] captured int8 gemm {M}x{N}x{K} layout {layout}", flush=True)
+    ctx = cap.ctx
+    assert ctx.plan_gemm_i8(M, N, K)["workgroups"] > workgroups  # run directly, it is split
+    A, B = synth.int8((M, K), 3), synth.int8((N, K) if layout == mi.B_NT else (K, N), 4)
+    want = oracle.gemm_i8_rq(A, B, 11, b_nt=layout == mi.B_NT)
+    dA, dB, dY = ctx.upload(A), ctx.upload(B), ctx.empty((M, N), np.int8)
+    exe, grids = cap.record(lambda: ctx.gemm_i8_rq(dA, dB, dY, M, N, K, 11, False, None, layout))
+    assert len(grids) == 1 and np.prod(grids[0]) == workgroups, grids
+
+    def check(rep):
+        assert np.array_equal(ctx.download(dY), want), rep
+
+    _beside_eager_splits(cap, exe, lambda: ctx.copy_h2d(dY, np.full((M, N), 77, np.int8)), check)
+    for b in (dA, dB, dY):
+        b.free()
+
+
+def test_captured_bf16_gemm_is_not_split(cap):
+    M, N, K = 130, 270, 1030
+    print(f"[case] captured bf16 gemm {M}x{N}x{K}", flush=True)
+    ctx = cap.ctx
+    A, B = synth.bf16_normal((M, K), 1, 1.0 / np.sqrt(K)), synth.bf16_normal((K, N), 2, 1.0)
+    R = oracle.gemm_bf16(A, B, f64=True)
+    dA, dB, dC = ctx.upload(A), ctx.upload(B), ctx.empty((M, N), np.float32)
+    exe, grids = cap.record(lambda: ctx.gemm_bf16_f32(dA, dB, dC, M, N, K))
+    assert len(grids) == 1 and grids[0][1] == 1, grids  # (the splits are in y)
+
+    def check(rep):
+        # K additions, each off by at most half an ulp of a partial sum, which
+        # stays below 6 times the results' rms
+        err = np.abs(ctx.download(dC).astype(np.float64) - R).max() / np.sqrt(np.mean(R * R))
+        assert err <= 6 * K * 2.0**-25, (rep, err)
+
+    _beside_eager_splits(cap, exe, lambda: ctx.copy_h2d(dC, np.full((M, N), np.nan, np.float32)), check)
+    for b in (dA, dB, dC):
+        b.free()
