@@ -223,7 +223,34 @@ __global__ __launch_bounds__(256) void fill_i8_kernel(int8_t* __restrict__ dst, 
 }  // namespace
 
 // ---------------------------------------------------------------- context
-extern "C" int miaie_init_on_stream(miaie_ctx** out, int device, void* stream) {
+namespace {
+
+// Zero device memory before any stream uses it, on a stream of its own: work
+// on the legacy stream would wait for every blocking stream, and would be
+// refused, and end the capture, while any stream of the process is captured.
+hipError_t clear_now(void* p, size_t bytes) {
+  hipStream_t st = nullptr;
+  hipError_t e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
+  if (e != hipSuccess) return e;
+  e = hipMemsetAsync(p, 0, bytes, st);
+  const hipError_t done = hipStreamSynchronize(st), gone = hipStreamDestroy(st);
+  return e != hipSuccess ? e : done != hipSuccess ? done : gone;
+}
+
+// Drop a context whose creation failed; returns rc.
+int discard(miaie_ctx* ctx, int rc) {
+  if (ctx->work) {
+    (void)dbg_remove(ctx, ctx->work);
+    (void)hipFree(ctx->work);
+  }
+  if (ctx->own_stream) (void)hipStreamDestroy(ctx->stream);
+  if (ctx->done) (void)hipEventDestroy(ctx->done);
+  delete ctx;
+  return rc;
+}
+
+// own: the context gets a stream of its own, else it launches onto `stream`.
+int create(miaie_ctx** out, int device, void* stream, bool own) {
   if (!out) return fail(nullptr, MIAIE_EINVAL, "miaie_init: ctx out-pointer is NULL");
   *out = nullptr;
   int count = 0;
@@ -245,69 +272,46 @@ extern "C" int miaie_init_on_stream(miaie_ctx** out, int device, void* stream) {
   ctx->id = next_id.fetch_add(1);
   ctx->device = device;
   ctx->cus = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 1;
-  if (stream) {
-    ctx->stream = static_cast<hipStream_t>(stream);
-  } else {
-    ctx->stream = nullptr;
-  }
+  ctx->stream = static_cast<hipStream_t>(stream);
   e = hipEventCreateWithFlags(&ctx->done, hipEventDisableTiming);
-  if (e != hipSuccess) {
-    int rc = hip_fail(nullptr, e, "hipEventCreate");
-    delete ctx;
-    return rc;
+  if (e != hipSuccess) return discard(ctx, hip_fail(nullptr, e, "hipEventCreate"));
+  if (own) {
+    e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
+    if (e != hipSuccess) return discard(ctx, hip_fail(nullptr, e, "hipStreamCreate"));
+    ctx->own_stream = true;
   }
   if (int rc = scratch_setup(ctx)) {
     fail(nullptr, rc, "%s", ctx->err);
-    (void)hipEventDestroy(ctx->done);
-    delete ctx;
-    return rc;
+    return discard(ctx, rc);
   }
   constexpr size_t kCounterBytes = MIAIE_CTX_COUNTERS * sizeof(uint32_t);
   e = hipMalloc(&ctx->work, MIAIE_CTX_WORK_BYTES + kCounterBytes);
-  if (e == hipSuccess) {
-    ctx->work_bytes = MIAIE_CTX_WORK_BYTES;
-    e = hipMemset(ctx_counters(ctx->work), 0, kCounterBytes);
-    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);  // done before any stream uses them
-  }
-  if (e != hipSuccess) {
-    int rc = hip_fail(nullptr, e, "hipMalloc (context workspace)");
-    if (ctx->work) (void)hipFree(ctx->work);
-    (void)hipEventDestroy(ctx->done);
-    delete ctx;
-    return rc;
-  }
+  if (e != hipSuccess) return discard(ctx, hip_fail(nullptr, e, "hipMalloc (context workspace)"));
+  ctx->work_bytes = MIAIE_CTX_WORK_BYTES;
+  // the arrival counters start at 0: in stream order on the context's own
+  // stream; a caller's stream may be one that is being captured
+  e = own ? hipMemsetAsync(ctx_counters(ctx->work), 0, kCounterBytes, ctx->stream)
+          : clear_now(ctx_counters(ctx->work), kCounterBytes);
+  if (e != hipSuccess) return discard(ctx, hip_fail(nullptr, e, "hipMemset (context workspace)"));
   // (debug build) the workspace and the scratch array are buffers the
   // kernels may touch
   int rc = dbg_add(ctx, ctx->work, ctx->work_bytes + kCounterBytes);
   if (rc == MIAIE_OK) rc = dbg_add(ctx, ctx->scratch, MIAIE_MLP_NOALLOC_MAX_H);
   if (rc != MIAIE_OK) {
     fail(nullptr, rc, "%s", ctx->err);
-    (void)dbg_remove(ctx, ctx->work);
-    (void)hipFree(ctx->work);
-    (void)hipEventDestroy(ctx->done);
-    delete ctx;
-    return rc;
+    return discard(ctx, rc);
   }
   *out = ctx;
   return MIAIE_OK;
 }
 
-extern "C" int miaie_init(miaie_ctx** out, int device) {
-  int rc = miaie_init_on_stream(out, device, nullptr);
-  if (rc != MIAIE_OK) return rc;
-  miaie_ctx* ctx = *out;
-  hipError_t e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
-  if (e != hipSuccess) {
-    rc = hip_fail(nullptr, e, "hipStreamCreate");
-    (void)hipFree(ctx->work);
-    (void)hipEventDestroy(ctx->done);
-    delete ctx;
-    *out = nullptr;
-    return rc;
-  }
-  ctx->own_stream = true;
-  return MIAIE_OK;
+}  // namespace
+
+extern "C" int miaie_init_on_stream(miaie_ctx** out, int device, void* stream) {
+  return create(out, device, stream, false);
 }
+
+extern "C" int miaie_init(miaie_ctx** out, int device) { return create(out, device, nullptr, true); }
 
 extern "C" int miaie_finish(miaie_ctx* ctx) {
   if (!ctx) return MIAIE_OK;

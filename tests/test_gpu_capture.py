@@ -3,6 +3,7 @@ stream (not miaie_graph_begin).  Such a graph may be replayed on any stream,
 beside other work of the context, so what it holds must not touch the
 context's workspace: no split of K."""
 import ctypes as C
+import threading
 
 import numpy as np
 import pytest
@@ -13,7 +14,7 @@ from aiehlc_amd import synth
 
 pytestmark = pytest.mark.gpu
 
-NON_BLOCKING, THREAD_LOCAL = 1, 1  # hipStreamNonBlocking, hipStreamCaptureModeThreadLocal
+NON_BLOCKING, THREAD_LOCAL, RELAXED = 1, 1, 2  # hipStreamNonBlocking, hipStreamCaptureMode*
 
 
 class _Dim3(C.Structure):
@@ -184,3 +185,57 @@ def test_captured_bf16_gemm_is_not_split(cap):
     _beside_eager_splits(cap, exe, lambda: ctx.copy_h2d(dC, np.full((M, N), np.nan, np.float32)), check)
     for b in (dA, dB, dC):
         b.free()
+
+
+@pytest.mark.parametrize("flags", [0, NON_BLOCKING])
+@pytest.mark.parametrize("mode", [THREAD_LOCAL, RELAXED])
+def test_a_context_is_created_while_another_thread_captures(cap, flags, mode):
+    """... on a stream of its own and on a caller's, neither of them nor the
+    capture fails, and they work (a split product uses the arrival counters)."""
+    print(f"[case] context created during a capture, stream flags {flags} mode {mode}", flush=True)
+    hip, begun, created, rcs = cap.hip, threading.Event(), threading.Event(), {}
+
+    def capture():
+        s, graph = C.c_void_p(), C.c_void_p()
+        rcs["device"] = hip.hipSetDevice(0)
+        rcs["stream"] = hip.hipStreamCreateWithFlags(C.byref(s), flags)
+        rcs["begin"] = hip.hipStreamBeginCapture(s, mode)
+        begun.set()
+        created.wait(60)
+        rcs["end"] = hip.hipStreamEndCapture(s, C.byref(graph))
+        hip.hipGraphDestroy(graph)
+        hip.hipStreamDestroy(s)
+
+    t = threading.Thread(target=capture)
+    t.start()
+    begun.wait(60)
+    made = []
+    try:
+        made = [mi.Context(0), mi.Context(0, stream=cap.streams[1].value)]
+    finally:
+        created.set()
+        t.join()
+    assert set(rcs.values()) == {0}, rcs
+    M, N, K = 16, 512, 8192
+    A, B = synth.int8((M, K), 1), synth.int8((K, N), 2)
+    for ctx in made:
+        dA, dB, dY = ctx.upload(A), ctx.upload(B), ctx.empty((M, N), np.int8)
+        ctx.gemm_i8_rq(dA, dB, dY, M, N, K, 11)
+        ctx.wait(60_000)
+        assert np.array_equal(ctx.download(dY), oracle.gemm_i8_rq(A, B, 11))
+        ctx.close()
+
+
+def test_a_context_is_created_by_the_capturing_thread(cap):
+    """In relaxed mode."""
+    hip, s, graph = cap.hip, C.c_void_p(), C.c_void_p()
+    cap.ok(hip.hipStreamCreateWithFlags(C.byref(s), NON_BLOCKING))
+    cap.ok(hip.hipStreamBeginCapture(s, RELAXED))
+    try:
+        mi.Context(0).close()
+        mi.Context(0, stream=cap.streams[1].value).close()
+    finally:
+        rc = hip.hipStreamEndCapture(s, C.byref(graph))
+    cap.ok(rc)
+    hip.hipGraphDestroy(graph)
+    cap.ok(hip.hipStreamDestroy(s))
