@@ -727,8 +727,8 @@ __global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void conv2d_i8_flex_walk(
   }
 }
 
-// Operands of fewer than 16 bytes, and above 2^31: one thread per output
-// element.
+// Operands of fewer than 16 bytes, and above 2^31, and more tiles than a launch
+// takes: one thread per output element.
 __global__ __launch_bounds__(256) void conv2d_i8_direct(const int8_t* __restrict__ X, const int8_t* __restrict__ W,
                                                         const uint8_t* __restrict__ shifts, int8_t* __restrict__ Y,
                                                         int N, int H, int Wd, int Cin, int Cout, int R, int S,
@@ -925,16 +925,22 @@ static bool flex_ok(int N, int H, int Wd, int Cin, int Cout, int R, int S, int p
          (R * cpr + 64) * cpr < ((size_t)1 << 32);
 }
 
-static int launch_flex(miaie_ctx* ctx, const int8_t* X, const int8_t* W, const uint8_t* shifts, int8_t* Y, int N, int H,
-                       int Wd, int Cin, int Cout, int R, int S, int stride, int pad, int Ho, int Wo) {
+// its tile and split (bm = 0: more tiles than a launch takes)
+static flex::Plan flex_plan(miaie_ctx* ctx, long P, int Cin, int Cout, int R, int S) {
+  const long k_bytes = 16l * R * ((S * Cin + 15) / 16);
+  const flex::Plan f = flex::plan(P, Cout, k_bytes, 1.5, ctx->cus, true, ctx->work_bytes);
+  return f.splits > 1 && !may_split(ctx) ? flex::plan(P, Cout, k_bytes, 1.5, ctx->cus, false, 0) : f;
+}
+
+static int launch_flex(miaie_ctx* ctx, const flex::Plan& f, const int8_t* X, const int8_t* W, const uint8_t* shifts,
+                       int8_t* Y, int N, int H, int Wd, int Cin, int Cout, int R, int S, int stride, int pad, int Ho,
+                       int Wo) {
   RunShape k{H, Wd, Cin, R, Ho, Wo, stride, pad, S * Cin, (S * Cin + 15) / 16, 0, 0, 0};
   auto inverse = [](int d) { return (uint32_t)(((uint64_t)1 << 32) / (uint64_t)d + 1); };
   k.cpr_inv = inverse(k.CPR);
   k.wo_inv = inverse(Wo);
   k.ho_inv = inverse(Ho);
   const long P = (long)N * Ho * Wo;
-  flex::Plan f = flex::plan(P, Cout, 16l * R * k.CPR, 1.5, ctx->cus, true, ctx->work_bytes);
-  if (f.splits > 1 && !may_split(ctx)) f = flex::plan(P, Cout, 16l * R * k.CPR, 1.5, ctx->cus, false, 0);
   hipError_t e = hipSuccess;
   flex::with_geom(f, [&](auto g) {
     using G = typename decltype(g)::type;
@@ -1026,8 +1032,10 @@ int launch_conv2d_i8(miaie_ctx* ctx, const int8_t* X, const int8_t* W, const uin
   // 8x64x64x160->512 1x1: 25.9 against 15.5; 2x56x56x64->64 stride 2, 25 tiles:
   // 4.7 against 6.8).
   const bool big = ((P + 63) / 64) * (size_t)((Cout + 63) / 64) >= 3 * (size_t)ctx->cus;
-  const bool flex = flex_ok(N, H, Wd, Cin, Cout, R, S, pad, P);
-  if (kernel == MIAIE_CONV_IGEMM && !(big && flex)) {
+  flex::Plan f;
+  if ((kernel != MIAIE_CONV_IGEMM || big) && flex_ok(N, H, Wd, Cin, Cout, R, S, pad, P))
+    f = flex_plan(ctx, (long)P, Cin, Cout, R, S);
+  if (kernel == MIAIE_CONV_IGEMM && !f.bm) {
     const unsigned pxb = (unsigned)((P + PIX - 1) / PIX), chb = (unsigned)(Cout / COB);
     if (ks > 1) {
       int32_t* const part = static_cast<int32_t*>(ctx->work);
@@ -1045,8 +1053,8 @@ int launch_conv2d_i8(miaie_ctx* ctx, const int8_t* X, const int8_t* W, const uin
                                                         Ho, Wo, 1);
     return check_launch(ctx, e, "conv2d_i8_igemm");
   }
-  if (flex) return launch_flex(ctx, X, W, shifts, Y, N, H, Wd, Cin, Cout, R, S, stride, pad, Ho, Wo);
-  // operands below 16 or above 2^31 bytes
+  if (f.bm) return launch_flex(ctx, f, X, W, shifts, Y, N, H, Wd, Cin, Cout, R, S, stride, pad, Ho, Wo);
+  // operands below 16 or above 2^31 bytes, or too many tiles
   const size_t total = P * Cout;
   const size_t blocks = (total + 255) / 256;
   if (blocks >= ((size_t)1 << 31)) return fail(ctx, MIAIE_EINVAL, "conv2d: output too large for the direct kernel");

@@ -91,6 +91,7 @@ struct Plan {
 // `cost`: stage cost relative to the int8 GEMM's (conv 1.5: its loads compute
 // their addresses).
 // (No divisions: this runs on the host for every call.)
+// bm is 0 where every tile makes too many workgroups for a launch.
 template <class G>
 inline void consider(Plan& best, double t0, double latency, double wg, double stage, double sum, double sum_split,
                      long M, long N, long k_bytes, double cost, int cus, double per_cu, bool can_split,
@@ -98,6 +99,7 @@ inline void consider(Plan& best, double t0, double latency, double wg, double st
   static constexpr int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16};
   static constexpr double kInverse[] = {1.0, 1.0 / 2, 1.0 / 3, 1.0 / 4, 1.0 / 6, 1.0 / 8, 1.0 / 12, 1.0 / 16};
   const long tiles = ((M + G::BM - 1) / G::BM) * ((N + G::BN - 1) / G::BN), stages = (k_bytes + G::KB - 1) / G::KB;
+  if (tiles >= 1l << 24) return;  // tiles are grid.x, in which HIP takes fewer than 2^32 threads
   const size_t slot = (size_t)tiles * G::BM * G::BN * sizeof(int32_t);
   auto up = [](double x) { return (double)(long)(x + (1.0 - 1e-6)); };  // rounded up
   for (int i = 0; i < 8; ++i) {

@@ -681,7 +681,7 @@ int launch_gemm_bf16(miaie_ctx* ctx, const uint16_t* A, const uint16_t* B, float
   // about 3 us and 0.0185 us per k (1024^3, 16 tiles: 23.6 us, 8.5 on 256 of
   // 64x64; 2048x4096x2048, 128 tiles: 43.1 us, as on 512 of 128x128).
   const double big_us = 3.0 + (double)((tiles + ctx->cus - 1) / ctx->cus) * (3.0 + 0.0185 * K);
-  if (big && (!flexible || big_us <= f.us)) {
+  if (big && (!f.bm || big_us <= f.us)) {
     if (K % (2 * BK) == 0)
       return check_launch(ctx, launch<gemm_bf16_pair16>(ctx->device, dim3(tiles), dim3(256), 0, ctx->stream, A, B, C, M, N, K),
                           "gemm_bf16_pair16");
@@ -689,7 +689,7 @@ int launch_gemm_bf16(miaie_ctx* ctx, const uint16_t* A, const uint16_t* B, float
                         "gemm_bf16_tile256");
   }
   if (grid.y > 65535) return fail(ctx, MIAIE_EINVAL, "gemm_bf16: M too large for the 64x64 fallback");
-  if (flexible) {
+  if (f.bm) {
     hipError_t e = hipSuccess;
     flex::with_geom(f, [&](auto g) {
       using G = typename decltype(g)::type;

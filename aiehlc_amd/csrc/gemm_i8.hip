@@ -448,7 +448,7 @@ static Route route(miaie_ctx* ctx, int M, int N, int K, bool pipe_ok, bool flex_
   if (r.pipe.bm != 256 && flex_ok) {
     r.flex = flex::plan(M, N, K, 1.0, ctx->cus, can_split, ctx->work_bytes);
     const double unit_us = (size_t)N * K > ((size_t)16 << 20) ? 0.7 : 0.5;
-    if (r.pipe.bm && K <= (1 << 15) && r.flex.us < 0.75 * (1.5 + unit_us * r.pipe.cost))
+    if (r.pipe.bm && r.flex.bm && K <= (1 << 15) && r.flex.us < 0.75 * (1.5 + unit_us * r.pipe.cost))
       r.pipe = PipePlan{};
     else if (r.pipe.bm)
       r.flex = flex::Plan{};
