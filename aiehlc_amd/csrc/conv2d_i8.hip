@@ -585,7 +585,7 @@ struct WeightLoader {
 // requantize outweigh the MFMAs.  8x48x48x96 -> 146, 5x5 (10 stages): 29 us,
 // 19.9 ms with one thread per output.
 template <class G>
-__global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void conv2d_i8_flex(const int8_t* __restrict__ X, const int8_t* __restrict__ W,
+__global__ __launch_bounds__(256, G::PER_CU) void conv2d_i8_flex(const int8_t* __restrict__ X, const int8_t* __restrict__ W,
                                                          const uint8_t* __restrict__ shifts, int8_t* __restrict__ Y,
                                                          RunShape k, int x_bytes, int P, int Cout,
                                                          int8_t* __restrict__ work, int splits) {
@@ -594,10 +594,11 @@ __global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void conv2d_i8_flex(const
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / G::WAVES_N, wn = wave % G::WAVES_N;
   int tm, tn;
-  miaie::dev::tile_coords<4>(blockIdx.x, (P + G::BM - 1) / G::BM, (Cout + G::BN - 1) / G::BN, tm, tn);
+  flex::tile_index<false>((P + G::BM - 1) / G::BM, (Cout + G::BN - 1) / G::BN, tm, tn);
   const int p0 = tm * G::BM, co0 = tn * G::BN;
   const int stages = (k.R * k.CPR + G::CH - 1) / G::CH, split = blockIdx.y;
-  const int s0 = (int)((long long)stages * split / splits), s1 = (int)((long long)stages * (split + 1) / splits);
+  int s0, s1;
+  flex::stage_range<G>(stages, split, splits, s0, s1);
 
   v4i acc[G::NI][G::NJ];
 #pragma unroll
@@ -615,7 +616,7 @@ __global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void conv2d_i8_flex(const
   PixelLoader<G, G::NA> la(X, k, x_bytes, p0, P, tid);
   WeightLoader<G, G::NB> lb(W, k, co0, Cout, tid);
   flex::tile_loop<int8_t, G, false>(lds, la, lb, s0, s1, lane, wm, wn, acc);
-  if (splits > 1 &&
+  if (G::SPLITS && splits > 1 &&
       !flex::split_sum<int8_t, G>(acc, blockIdx.x, split, splits, work, miaie::ctx_counters(work), &flag, tid))
     return;
 
@@ -653,7 +654,7 @@ struct WalkGeom {
   static constexpr int LDS = G::A_BYTES + G::B_BYTES + G::BM * G::YP;
 };
 template <class G>
-__global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void conv2d_i8_flex_walk(
+__global__ __launch_bounds__(256, G::PER_CU) void conv2d_i8_flex_walk(
     const int8_t* __restrict__ X, const int8_t* __restrict__ W, const uint8_t* __restrict__ shifts,
     int8_t* __restrict__ Y, RunShape k, int x_bytes, int P, int Cout, int step, int dn, int dh, int dw) {
   __shared__ __attribute__((aligned(1024))) int8_t lds[WalkGeom<G>::LDS];
@@ -949,7 +950,7 @@ static int launch_flex(miaie_ctx* ctx, const flex::Plan& f, const int8_t* X, con
     // that fit (by LDS and registers, 4 per CU, 2 of 128x128).  (Fewer
     // workgroups, each with the same number of tiles: 12.7 us against 11.3 for
     // 8x224x224x3 -> 64, 7x7, stride 2.)
-    const long step = std::max(1l, (G::BM < 128 ? 4l : 2l) * ctx->cus / tn);
+    const long step = std::max(1l, (long)G::PER_CU * ctx->cus / tn);
     if (16 * R * k.CPR <= G::KB && tm > step) {
       const long pixels = step * G::BM;  // from one of a workgroup's tiles to its next
       e = launch<conv2d_i8_flex_walk<G>>(ctx->device, dim3((unsigned)(tn * step)), dim3(256), 0, ctx->stream, X, W,

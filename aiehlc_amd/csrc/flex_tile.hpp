@@ -13,7 +13,7 @@
 // together) while the current stage, in LDS, is multiplied on
 // v_mfma_i32_16x16x64_i8 / v_mfma_f32_16x16x32_bf16.  What bounds such small
 // products is the latency of that chain of loads, so a stage is as deep as the
-// registers allow (256 bytes of k: a product of K = 1000 is 4 stages), 2-4
+// registers allow (256 bytes of k: a product of K = 1000 is 4 stages), 2-8
 // workgroups share a CU, and K is split over workgroups where tiles are few.
 //
 // Loads are 16 bytes wide from any byte address (gfx950's unaligned access
@@ -64,18 +64,24 @@ struct Geom {
   static constexpr int A_BYTES = BM * KB, B_BYTES = BN * KB;
   static constexpr int NA = A_BYTES / 4096, NB = B_BYTES / 4096;  // chunks per thread per stage
   static constexpr int YP = BN + 16;                         // LDS pitch of an int8 output row
+  static constexpr bool SPLITS = KB >= 128;  // whether its K is ever split
+  static constexpr int PER_CU = BM >= 128 ? 2 : KB < 256 ? 8 : 4;  // workgroups whose registers and LDS fit a CU
   static constexpr int LDS = A_BYTES + B_BYTES > BM * YP ? A_BYTES + B_BYTES : BM * YP;
   static_assert(NA >= 1 && NB >= 1 && NI >= 1 && NJ >= 1, "tile too small for 4 waves");
 };
 
-// The tiles in use: few rows; small and ragged products; large ones.
+// The tiles in use: a k of a few chunks; few rows; small and ragged products;
+// large ones.  (A stage is loaded, written to LDS and multiplied whole: 16 to 128
+// bytes of k in a 256-byte stage took 3.0 us where 2.5 suffice for 16x16x16 bf16,
+// 5.4 against 3.7 for int8 65000x16x16 NT.)
+using Short = Geom<64, 64, 64, 2>;
 using Skinny = Geom<16, 128, 256, 4>;
 using Small = Geom<64, 64, 256, 2>;
 using Large = Geom<128, 128, 128, 2>;
 
 // Output tile and workgroups per tile for an M x N product of k_bytes of k.
 struct Plan {
-  int bm = 0, bn = 0, splits = 1;
+  int bm = 0, bn = 0, kb = 0, splits = 1;
   long tiles = 0;  // workgroups = tiles * splits
   double us = 0;   // estimated time
 };
@@ -109,12 +115,15 @@ inline void consider(Plan& best, double t0, double latency, double wg, double st
       return;
     const double n = up((double)stages * kInverse[i]), rounds = up((double)(tiles * s) * per_cu);
     const double us = t0 + std::max(latency * cost * n, rounds * (wg + stage * cost * n)) + (s > 1 ? sum + sum_split * s : 0.0);
-    if (best.bm == 0 || us < best.us) best = Plan{G::BM, G::BN, s, tiles, us};
+    if (best.bm == 0 || us < best.us) best = Plan{G::BM, G::BN, G::KB, s, tiles, us};
   }
 }
 inline Plan plan(long M, long N, long k_bytes, double cost, int cus, bool can_split, size_t work_bytes) {
   Plan best;
   const double per_cu = 1.0 / cus;
+  // (a k of three 64-byte stages at most: longer ones gain by deeper stages)
+  if (k_bytes * cost <= 192)
+    consider<Short>(best, 2.35, 0.40, 0.18, 0.19, 0.0, 0.0, M, N, k_bytes, cost, cus, per_cu, false, work_bytes);
   consider<Skinny>(best, 1.7, 0.95, 0.90, 0.80, 1.6, 0.15, M, N, k_bytes, cost, cus, per_cu, can_split, work_bytes);
   consider<Small>(best, 2.4, 0.84, 0.55, 0.50, 1.5, 0.26, M, N, k_bytes, cost, cus, per_cu, can_split, work_bytes);
   consider<Large>(best, 3.5, 0.95, 1.20, 0.60, 1.5, 1.00, M, N, k_bytes, cost, cus, per_cu, can_split, work_bytes);
@@ -124,7 +133,9 @@ inline Plan plan(long M, long N, long k_bytes, double cost, int cus, bool can_sp
 // Calls go with the geometry a plan names, as a type.
 template <class F>
 void with_geom(const Plan& p, F&& go) {
-  if (p.bm == Skinny::BM)
+  if (p.kb == Short::KB)
+    go(type_t<Short>{});
+  else if (p.bm == Skinny::BM)
     go(type_t<Skinny>{});
   else if (p.bm == Small::BM)
     go(type_t<Small>{});
@@ -296,11 +307,27 @@ struct ColsLoader {
 template <bool PAIRS>
 __device__ __forceinline__ void tile_index(int TM, int TN, int& tm, int& tn) {
   const int b = blockIdx.x;
-  if (PAIRS && TM == 1) {
+  if (TN == 1) {  // (tile_coords' order, without its divisions)
+    tm = TM % 8 == 0 ? (b & 7) * (TM >> 3) + (b >> 3) : b;
+    tn = 0;
+  } else if (PAIRS && TM == 1) {
     tm = 0;
     tn = (b | 15) < TN ? (b & ~15) + 2 * (b & 7) + ((b >> 3) & 1) : b;
   } else {
     dev::tile_coords<4>(b, TM, TN, tm, tn);
+  }
+}
+
+// The stages [s0, s1) of one of the `splits` workgroups of a tile.  (32 bits
+// hold 16 splits of 2^24 stages; in 64 bits the two divisions were 400 scalar
+// instructions ahead of the first load.)
+template <class G>
+__device__ __forceinline__ void stage_range(int stages, int split, int splits, int& s0, int& s1) {
+  s0 = 0;
+  s1 = stages;
+  if (G::SPLITS && splits > 1) {
+    s0 = (int)((uint32_t)stages * (uint32_t)split / (uint32_t)splits);
+    s1 = (int)((uint32_t)stages * (uint32_t)(split + 1) / (uint32_t)splits);
   }
 }
 
@@ -379,6 +406,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t device_buffer(void* p, int byt
 template <class T, class G>
 __device__ __forceinline__ bool split_sum(typename Mma<T>::acc_t (&acc)[G::NI][G::NJ], int tile, int split, int splits,
                                           int8_t* work, uint32_t* counters, int* flag, int tid) {
+  if constexpr (!G::SPLITS) return true;
   using acc_t = typename Mma<T>::acc_t;
   constexpr int TILE = G::BM * G::BN / 4;  // accumulator vectors per tile
   acc_t* const slots = reinterpret_cast<acc_t*>(work) + (size_t)tile * splits * TILE;

@@ -623,7 +623,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_tile64(const uint16_t* __restri
 // chain of their loads): 9.4 us, 25.1 in a 64x64 kernel with one 32-wide k-step
 // in flight; 256x4096x2048: 13.7 us split in 2, 40.8 on 16 tiles of 256x256.
 template <class G>
-__global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void gemm_bf16_flex(const uint16_t* __restrict__ A,
+__global__ __launch_bounds__(256, G::PER_CU) void gemm_bf16_flex(const uint16_t* __restrict__ A,
                                                          const uint16_t* __restrict__ B, float* __restrict__ C,
                                                          int M, int N, int K, int8_t* __restrict__ work, int splits) {
   __shared__ __attribute__((aligned(1024))) int8_t lds[G::LDS];
@@ -631,10 +631,11 @@ __global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void gemm_bf16_flex(const
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / G::WAVES_N, wn = wave % G::WAVES_N;
   int tm, tn;
-  dev::tile_coords<4>(blockIdx.x, (M + G::BM - 1) / G::BM, (N + G::BN - 1) / G::BN, tm, tn);
+  flex::tile_index<false>((M + G::BM - 1) / G::BM, (N + G::BN - 1) / G::BN, tm, tn);
   const int m0 = tm * G::BM, n0 = tn * G::BN;
   const int stages = (2 * K + G::KB - 1) / G::KB, split = blockIdx.y;
-  const int s0 = (int)((long long)stages * split / splits), s1 = (int)((long long)stages * (split + 1) / splits);
+  int s0, s1;
+  flex::stage_range<G>(stages, split, splits, s0, s1);
 
   v4f acc[G::NI][G::NJ];
 #pragma unroll
@@ -644,7 +645,7 @@ __global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void gemm_bf16_flex(const
   flex::RowsLoader<G, G::NA> la(reinterpret_cast<const int8_t*>(A), m0, M, (size_t)K * 2, 2 * K, tid);
   flex::ColsLoader<uint16_t, G, true> lb(reinterpret_cast<const int8_t*>(B), n0, N, (size_t)N * 2, K, tid);
   flex::tile_loop<uint16_t, G, true>(lds, la, lb, s0, s1, lane, wm, wn, acc);
-  if (splits > 1 &&
+  if (G::SPLITS && splits > 1 &&
       !flex::split_sum<uint16_t, G>(acc, blockIdx.x, split, splits, work, miaie::ctx_counters(work), &flag, tid))
     return;
 

@@ -139,16 +139,17 @@ __global__ __launch_bounds__(256) void gemm_i8_tile64(const int8_t* __restrict__
 // Register-staged tiles (flex_tile.hpp): any size, stride and alignment with
 // rows of at least 16 bytes.  grid.x: output tiles, grid.y: the `splits`
 // workgroups that divide a tile's K; mode: shift, relu << 8, splits << 16 (one
-// argument: each costs the launch host time).  Bound by the latency of the stages'
+// argument: each costs the launch host time; what the loads need comes first,
+// in the 14 dwords that arrive in SGPRs).  Bound by the latency of the stages'
 // loads, and for few rows by reading B: 1000 x 2050 x 1000 NT (rows of 1000
 // bytes) took 61.1 us in the byte-wise 64x64 kernel and takes 8.8; the MLP
 // over 16 rows (4096 -> 11008 -> 4096, 90 MB of weights) 204.7 us in a
 // vectorised 64x64 kernel without a split and 29.2 (27.3 with K split 8
 // ways, 72 unsplit, on one box).
 template <class G, bool B_NT>
-__global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void gemm_i8_flex(const int8_t* __restrict__ A, const int8_t* __restrict__ B,
-                                                       int8_t* __restrict__ Y, int32_t* __restrict__ C, int M, int N,
-                                                       int K, int lda, int ldb, int ldy, int ldc, uint32_t mode,
+__global__ __launch_bounds__(256, G::PER_CU) void gemm_i8_flex(const int8_t* __restrict__ A, const int8_t* __restrict__ B, int M,
+                                                       int N, int K, int lda, int ldb, uint32_t mode,
+                                                       int8_t* __restrict__ Y, int32_t* __restrict__ C, int ldy, int ldc,
                                                        int8_t* __restrict__ work) {
   const int shift = mode & 31, relu = (mode >> 8) & 1, splits = mode >> 16;
   __shared__ __attribute__((aligned(1024))) int8_t lds[G::LDS];
@@ -159,7 +160,8 @@ __global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void gemm_i8_flex(const i
   flex::tile_index<!B_NT && G::BN == 64>((M + G::BM - 1) / G::BM, (N + G::BN - 1) / G::BN, tm, tn);
   const int m0 = tm * G::BM, n0 = tn * G::BN;
   const int stages = (K + G::KB - 1) / G::KB, split = blockIdx.y;
-  const int s0 = (int)((long long)stages * split / splits), s1 = (int)((long long)stages * (split + 1) / splits);
+  int s0, s1;
+  flex::stage_range<G>(stages, split, splits, s0, s1);
 
   v4i acc[G::NI][G::NJ];
 #pragma unroll
@@ -174,7 +176,7 @@ __global__ __launch_bounds__(256, G::BM < 128 ? 4 : 2) void gemm_i8_flex(const i
     flex::ColsLoader<int8_t, G, false> lb(B, n0, N, ldb, K, tid);
     flex::tile_loop<int8_t, G, true>(lds, la, lb, s0, s1, lane, wm, wn, acc);
   }
-  if (splits > 1 &&
+  if (G::SPLITS && splits > 1 &&
       !flex::split_sum<int8_t, G>(acc, blockIdx.x, split, splits, work, miaie::ctx_counters(work), &flag, tid))
     return;
 
@@ -526,10 +528,10 @@ int launch_gemm_i8(miaie_ctx* ctx, const int8_t* A, const int8_t* B, int8_t* Y, 
       const dim3 fg((unsigned)f.tiles, (unsigned)f.splits);
       int8_t* const work = static_cast<int8_t*>(ctx->work);
       const uint32_t mode = (uint32_t)(shift | relu << 8 | f.splits << 16);
-      e = b_nt ? launch<gemm_i8_flex<G, true>>(dev, fg, block, 0, ctx->stream, A, B, Y, C, M, N, K, lda, ldb, ldy, ldc,
-                                               mode, work)
-               : launch<gemm_i8_flex<G, false>>(dev, fg, block, 0, ctx->stream, A, B, Y, C, M, N, K, lda, ldb, ldy, ldc,
-                                                mode, work);
+      e = b_nt ? launch<gemm_i8_flex<G, true>>(dev, fg, block, 0, ctx->stream, A, B, M, N, K, lda, ldb, mode, Y, C,
+                                               ldy, ldc, work)
+               : launch<gemm_i8_flex<G, false>>(dev, fg, block, 0, ctx->stream, A, B, M, N, K, lda, ldb, mode, Y, C,
+                                                ldy, ldc, work);
     });
     return check_launch(ctx, e, "gemm_i8_flex");
   }

@@ -17,6 +17,10 @@ def _i8(rng, *shape):
     return rng.integers(-128, 128, size=shape, dtype=np.int8)
 
 
+# K at the edges of the short tile's 64-byte stages, of which it takes three
+SHORT_K = [(M, N, K) for K in (16, 31, 63, 64, 65, 127, 128, 129, 191, 192, 193)
+           for M, N in ((1, 17), (65, 63), (64, 130), (700, 40))]
+
 GEMM_SHAPES = [
     # M, N, K
     (1, 16, 16),      # the smallest that runs here: one chunk of one row
@@ -37,7 +41,7 @@ GEMM_SHAPES = [
 ]
 
 
-@pytest.mark.parametrize("M,N,K", GEMM_SHAPES)
+@pytest.mark.parametrize("M,N,K", GEMM_SHAPES + SHORT_K)
 @pytest.mark.parametrize("layout", [mi.B_NN, mi.B_NT])
 def test_gemm_i8_flex(ctx, M, N, K, layout):
     print(f"[case] flex gemm {M}x{N}x{K} layout {layout} plan {ctx.plan_gemm_i8(M, N, K)}", flush=True)
@@ -151,7 +155,7 @@ BF16_SHAPES = [
 ]
 
 
-@pytest.mark.parametrize("M,N,K", BF16_SHAPES)
+@pytest.mark.parametrize("M,N,K", BF16_SHAPES + [(M, N, (K + 1) // 2) for M, N, K in SHORT_K])
 def test_gemm_bf16_flex(ctx, M, N, K):
     print(f"[case] flex bf16 {M}x{N}x{K}", flush=True)
     A = synth.bf16_normal((M, K), 1, 1.0 / np.sqrt(K))
@@ -232,6 +236,11 @@ CONV_SHAPES = [
     (4, 64, 64, 3, 130, 3, 3, 1, 1),  # 256 x 2 tiles: 128 x 128
     (8, 96, 96, 32, 192, 1, 1, 1, 0),  # a large grid of the implicit-GEMM shapes
     # one stage of k and more pixel tiles than fit at once: walked over
+    (1, 520, 262, 3, 20, 3, 3, 1, 1),   # rows longer than a tile; k of 48 bytes
+    (4100, 6, 7, 3, 10, 3, 3, 1, 1),    # images smaller than a tile
+    (1, 260, 262, 3, 20, 7, 7, 1, 3),   # k of 224 bytes: 256-byte stages
+    (8, 160, 160, 100, 128, 1, 1, 1, 0),  # 128 x 128
+    # (fewer tiles than fit with 64-byte stages)
     (1, 260, 262, 3, 20, 3, 3, 1, 1),   # rows longer than a tile
     (2100, 6, 7, 3, 10, 3, 3, 1, 1),    # images smaller than a tile
     (70000, 2, 1, 16, 70, 1, 1, 1, 0),  # one column, two channel tiles, the last partial
