@@ -36,6 +36,7 @@
 #pragma once
 
 #include <algorithm>
+#include <type_traits>
 
 #include "gfx950_ops.hpp"
 #include "miaie_internal.hpp"
@@ -82,6 +83,7 @@ using Large = Geom<128, 128, 128, 2>;
 // Output tile and workgroups per tile for an M x N product of k_bytes of k.
 struct Plan {
   int bm = 0, bn = 0, kb = 0, splits = 1;
+  bool any = false;  // rows of B below 16 bytes, or a pitch of 2^25 or more
   long tiles = 0;  // workgroups = tiles * splits
   double us = 0;   // estimated time
 };
@@ -115,19 +117,39 @@ inline void consider(Plan& best, double t0, double latency, double wg, double st
       return;
     const double n = up((double)stages * kInverse[i]), rounds = up((double)(tiles * s) * per_cu);
     const double us = t0 + std::max(latency * cost * n, rounds * (wg + stage * cost * n)) + (s > 1 ? sum + sum_split * s : 0.0);
-    if (best.bm == 0 || us < best.us) best = Plan{G::BM, G::BN, G::KB, s, tiles, us};
+    if (best.bm == 0 || us < best.us) best = Plan{G::BM, G::BN, G::KB, s, false, tiles, us};
   }
 }
-inline Plan plan(long M, long N, long k_bytes, double cost, int cus, bool can_split, size_t work_bytes) {
-  Plan best;
+template <class G>
+inline void consider_tile(Plan& best, long M, long N, long k_bytes, double cost, int cus, bool can_split, size_t work_bytes) {
   const double per_cu = 1.0 / cus;
-  // (a k of three 64-byte stages at most: longer ones gain by deeper stages)
-  if (k_bytes * cost <= 192)
-    consider<Short>(best, 2.35, 0.40, 0.18, 0.19, 0.0, 0.0, M, N, k_bytes, cost, cus, per_cu, false, work_bytes);
-  consider<Skinny>(best, 1.7, 0.95, 0.90, 0.80, 1.6, 0.15, M, N, k_bytes, cost, cus, per_cu, can_split, work_bytes);
-  consider<Small>(best, 2.4, 0.84, 0.55, 0.50, 1.5, 0.26, M, N, k_bytes, cost, cus, per_cu, can_split, work_bytes);
-  consider<Large>(best, 3.5, 0.95, 1.20, 0.60, 1.5, 1.00, M, N, k_bytes, cost, cus, per_cu, can_split, work_bytes);
+  if constexpr (std::is_same_v<G, Short>) {
+    // (a k of three 64-byte stages at most: longer ones gain by deeper stages)
+    if (k_bytes * cost <= 192)
+      consider<G>(best, 2.35, 0.40, 0.18, 0.19, 0.0, 0.0, M, N, k_bytes, cost, cus, per_cu, false, work_bytes);
+  } else if constexpr (std::is_same_v<G, Skinny>) {
+    consider<G>(best, 1.7, 0.95, 0.90, 0.80, 1.6, 0.15, M, N, k_bytes, cost, cus, per_cu, can_split, work_bytes);
+  } else if constexpr (std::is_same_v<G, Small>) {
+    consider<G>(best, 2.4, 0.84, 0.55, 0.50, 1.5, 0.26, M, N, k_bytes, cost, cus, per_cu, can_split, work_bytes);
+  } else {
+    consider<G>(best, 3.5, 0.95, 1.20, 0.60, 1.5, 1.00, M, N, k_bytes, cost, cus, per_cu, can_split, work_bytes);
+  }
+}
+template <class... G>
+inline Plan plan_of(long M, long N, long k_bytes, double cost, int cus, bool can_split, size_t work_bytes) {
+  Plan best;
+  (consider_tile<G>(best, M, N, k_bytes, cost, cus, can_split, work_bytes), ...);
   return best;
+}
+inline Plan plan(long M, long N, long k_bytes, double cost, int cus, bool can_split, size_t work_bytes) {
+  return plan_of<Short, Skinny, Small, Large>(M, N, k_bytes, cost, cus, can_split, work_bytes);
+}
+// The same for the loaders that take any operand (with_geom_any), on 64 x 64
+// tiles alone.
+inline Plan plan_any(long M, long N, long k_bytes, int cus, bool can_split, size_t work_bytes) {
+  Plan p = plan_of<Short, Small>(M, N, k_bytes, 1.0, cus, can_split, work_bytes);
+  p.any = p.bm != 0;
+  return p;
 }
 
 // Calls go with the geometry a plan names, as a type.
@@ -141,6 +163,14 @@ void with_geom(const Plan& p, F&& go) {
     go(type_t<Small>{});
   else
     go(type_t<Large>{});
+}
+
+template <class F>
+void with_geom_any(const Plan& p, F&& go) {
+  if (p.kb == Short::KB)
+    go(type_t<Short>{});
+  else
+    go(type_t<Small>{});
 }
 
 __device__ __forceinline__ int row_off(int KB, int row, int chunk) {
@@ -215,11 +245,11 @@ __device__ __forceinline__ v4i byte_mask(int lo, int hi) {
 // chunks, set right where they reached past an end, into LDS.
 
 // Rows of a k-contiguous operand: chunk ch of rows r0 + RPP i of the tile,
-// zero past the last k.  k_bytes >= 16, pitch below 2^25.
-template <class G, int NL>
+// zero past the last k.  k_bytes >= 16; with 32-bit offsets, pitch below 2^25.
+template <class G, int NL, class Off = uint32_t>
 struct RowsLoader {
   const int8_t* base;  // first row of the tile
-  uint32_t voff[NL];
+  Off voff[NL];
   int k_bytes, r0, ch;
   v4i v[NL];
   // tile rows row0 .. of an operand of `rows` rows of k_bytes_ bytes, pitch ld
@@ -227,7 +257,7 @@ struct RowsLoader {
   __device__ __forceinline__ RowsLoader(const int8_t* p, int row0, int rows, size_t ld, int k_bytes_, int tid)
       : base(p + (size_t)row0 * ld), k_bytes(k_bytes_), r0(tid / G::CH), ch(tid % G::CH) {
 #pragma unroll
-    for (int i = 0; i < NL; ++i) voff[i] = (uint32_t)min(r0 + G::RPP * i, rows - 1 - row0) * (uint32_t)ld;
+    for (int i = 0; i < NL; ++i) voff[i] = (Off)min(r0 + G::RPP * i, rows - 1 - row0) * (Off)ld;
   }
   __device__ __forceinline__ void load(int s) {
     const uint32_t at = (uint32_t)min(s * G::KB + 16 * ch, k_bytes - 16);
@@ -291,6 +321,41 @@ struct ColsLoader {
 #pragma unroll
     for (int i = 0; i < G::NB; ++i) {
       const int k = k0 + KPP * i;
+      *reinterpret_cast<v4i*>(lds + k * PB + ((cb ^ kswz<T, PB>(k)) << 4)) = v[i];
+    }
+  }
+};
+
+// The same for any N >= 1 and pitch, where the whole operand is 16 bytes or
+// more: rows narrower than a load, too.  A chunk is loaded from where it starts
+// (past the end of its row it holds the next one's values), or from the
+// operand's last 16 bytes and shifted.
+template <class T, class G, bool ZERO>
+struct ColsLoaderAny {
+  static constexpr int PB = G::BN * (int)sizeof(T);
+  static constexpr int CB = PB / 16, KPP = 256 / CB;
+  static constexpr int SK = G::KB / (int)sizeof(T);
+  const int8_t* base;
+  size_t ld, want, last;  // first byte of the chunk in its row, last offset a load may start at
+  int K, k0, cb;
+  v4i v[G::NB];
+  int moved[G::NB];
+  __device__ __forceinline__ ColsLoaderAny(const int8_t* p, int n0, int N, size_t ld_, int K_, int tid)
+      : base(p), ld(ld_), want((size_t)n0 * sizeof(T) + 16 * (tid % CB)),
+        last((size_t)(K_ - 1) * ld_ + (size_t)N * sizeof(T) - 16), K(K_), k0(tid / CB), cb(tid % CB) {}
+  __device__ __forceinline__ void load(int s) {
+#pragma unroll
+    for (int i = 0; i < G::NB; ++i) {
+      const size_t at = (size_t)min(s * SK + k0 + KPP * i, K - 1) * ld + want, from = at < last ? at : last;
+      v[i] = MIAIE_LD(reinterpret_cast<const Any16*>(base + from)).v;
+      moved[i] = at - from < 16 ? (int)(at - from) : 16;
+    }
+  }
+  __device__ __forceinline__ void put(int s, int8_t* lds) {
+#pragma unroll
+    for (int i = 0; i < G::NB; ++i) {
+      const int k = k0 + KPP * i;
+      v[i] = ZERO && s * SK + k >= K ? v4i{0} : shr_bytes(v[i], moved[i]);
       *reinterpret_cast<v4i*>(lds + k * PB + ((cb ^ kswz<T, PB>(k)) << 4)) = v[i];
     }
   }

@@ -17,9 +17,9 @@
 //   gemm_bf16_tile256  256x256x32, 4 waves x (4x4 MFMA 32x32x16), four LDS stages.
 //   gemm_bf16_flex     register-staged 16x128, 64x64 and 128x128 tiles
 //                      (flex_tile.hpp) for every other size and alignment with
-//                      rows of at least 16 bytes, and wherever 256x256 tiles
-//                      are too few; K split over workgroups.
-//   gemm_bf16_tile64   64x64x32, bounds-checked, for rows below 16 bytes.
+//                      K >= 8, and wherever 256x256 tiles are too few; K split
+//                      over workgroups.
+//   gemm_bf16_tile64   64x64x32, bounds-checked, for K < 8.
 // The 256x256 kernels write C through whole-row stores staged in LDS.
 #include <type_traits>
 
@@ -617,12 +617,14 @@ __global__ __launch_bounds__(256) void gemm_bf16_tile64(const uint16_t* __restri
   }
 }
 
-// Register-staged tiles (flex_tile.hpp): any size and alignment with rows of
-// at least 16 bytes.  grid.x: output tiles, grid.y: the `splits` workgroups
-// that divide a tile's K.  1000^3 (256 tiles of 64x64, 8 stages, bound by the
-// chain of their loads): 9.4 us, 25.1 in a 64x64 kernel with one 32-wide k-step
-// in flight; 256x4096x2048: 13.7 us split in 2, 40.8 on 16 tiles of 256x256.
-template <class G>
+// Register-staged tiles (flex_tile.hpp): any size and alignment with K >= 8.
+// grid.x: output tiles, grid.y: the `splits` workgroups that divide a tile's K.
+// 1000^3 (256 tiles of 64x64, 8 stages, bound by the chain of their loads): 9.4
+// us, 25.1 in a 64x64 kernel with one 32-wide k-step in flight; 256x4096x2048:
+// 13.7 us split in 2, 40.8 on 16 tiles of 256x256.
+// ANY: 64-bit offsets and a B of any width (64x64 tiles alone): 4096x7x4096
+// 13.6 us, 80 in a vectorised 64x64 kernel without a split.
+template <class G, bool ANY>
 __global__ __launch_bounds__(256, G::PER_CU) void gemm_bf16_flex(const uint16_t* __restrict__ A,
                                                          const uint16_t* __restrict__ B, float* __restrict__ C,
                                                          int M, int N, int K, int8_t* __restrict__ work, int splits) {
@@ -642,8 +644,10 @@ __global__ __launch_bounds__(256, G::PER_CU) void gemm_bf16_flex(const uint16_t*
   for (int i = 0; i < G::NI; ++i)
 #pragma unroll
     for (int j = 0; j < G::NJ; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-  flex::RowsLoader<G, G::NA> la(reinterpret_cast<const int8_t*>(A), m0, M, (size_t)K * 2, 2 * K, tid);
-  flex::ColsLoader<uint16_t, G, true> lb(reinterpret_cast<const int8_t*>(B), n0, N, (size_t)N * 2, K, tid);
+  using Off = std::conditional_t<ANY, size_t, uint32_t>;
+  using Cols = std::conditional_t<ANY, flex::ColsLoaderAny<uint16_t, G, true>, flex::ColsLoader<uint16_t, G, true>>;
+  flex::RowsLoader<G, G::NA, Off> la(reinterpret_cast<const int8_t*>(A), m0, M, (size_t)K * 2, 2 * K, tid);
+  Cols lb(reinterpret_cast<const int8_t*>(B), n0, N, (size_t)N * 2, K, tid);
   flex::tile_loop<uint16_t, G, true>(lds, la, lb, s0, s1, lane, wm, wn, acc);
   if (G::SPLITS && splits > 1 &&
       !flex::split_sum<uint16_t, G>(acc, blockIdx.x, split, splits, work, miaie::ctx_counters(work), &flag, tid))
@@ -669,14 +673,18 @@ int launch_gemm_bf16(miaie_ctx* ctx, const uint16_t* A, const uint16_t* B, float
   const long tiles = (long)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
   const bool big = M >= BM && N >= BN && N % 8 == 0 && K % BK == 0 && aligned(A, 16) && aligned(B, 16) &&
                    aligned(C, 16) && K < (1 << 24) && N < (1 << 24);
-  // Register-staged tiles: rows of at least 16 bytes, and 32-bit offsets
-  // within a tile.
-  const bool flexible = K >= 8 && N >= 8 && K < (1 << 24) && N < (1 << 24);
+  // Register-staged tiles: rows of at least 16 bytes and 32-bit offsets within
+  // a tile, or (any) rows of A of 16 bytes alone.
+  const bool any = N < 8 || K >= (1 << 24) || N >= (1 << 24);
   const dim3 grid((N + 63) / 64, (M + 63) / 64);
+  auto flex_plan = [&](bool can_split) {
+    return any ? flex::plan_any(M, N, 2l * K, ctx->cus, can_split, ctx->work_bytes)
+               : flex::plan(M, N, 2l * K, 1.0, ctx->cus, can_split, ctx->work_bytes);
+  };
   flex::Plan f;
-  if (flexible) {
-    f = flex::plan(M, N, 2l * K, 1.0, ctx->cus, true, ctx->work_bytes);
-    if (f.splits > 1 && !may_split(ctx)) f = flex::plan(M, N, 2l * K, 1.0, ctx->cus, false, 0);
+  if (K >= 8 && K < (1 << 29) && N < (1 << 29)) {
+    f = flex_plan(true);
+    if (f.splits > 1 && !may_split(ctx)) f = flex_plan(false);
   }
   // Where both apply, the one estimated faster: a round of 256x256 tiles takes
   // about 3 us and 0.0185 us per k (1024^3, 16 tiles: 23.6 us, 8.5 on 256 of
@@ -692,11 +700,14 @@ int launch_gemm_bf16(miaie_ctx* ctx, const uint16_t* A, const uint16_t* B, float
   if (grid.y > 65535) return fail(ctx, MIAIE_EINVAL, "gemm_bf16: M too large for the 64x64 fallback");
   if (f.bm) {
     hipError_t e = hipSuccess;
-    flex::with_geom(f, [&](auto g) {
-      using G = typename decltype(g)::type;
-      e = launch<gemm_bf16_flex<G>>(ctx->device, dim3((unsigned)f.tiles, (unsigned)f.splits), dim3(256), 0, ctx->stream,
-                                    A, B, C, M, N, K, static_cast<int8_t*>(ctx->work), f.splits);
-    });
+    auto go = [&](auto k) {
+      e = launch<decltype(k)::value>(ctx->device, dim3((unsigned)f.tiles, (unsigned)f.splits), dim3(256), 0, ctx->stream,
+                                     A, B, C, M, N, K, static_cast<int8_t*>(ctx->work), f.splits);
+    };
+    if (f.any)
+      flex::with_geom_any(f, [&](auto g) { go(kernel_t<gemm_bf16_flex<typename decltype(g)::type, true>>{}); });
+    else
+      flex::with_geom(f, [&](auto g) { go(kernel_t<gemm_bf16_flex<typename decltype(g)::type, false>>{}); });
     return check_launch(ctx, e, "gemm_bf16_flex");
   }
   return check_launch(ctx, launch<gemm_bf16_tile64>(ctx->device, grid, dim3(256), 0, ctx->stream, A, B, C, M, N, K),

@@ -25,9 +25,9 @@
 //                   tiles in one launch.
 //   gemm_i8_flex    register-staged 16x128, 64x64 and 128x128 tiles
 //                   (flex_tile.hpp) for every other shape, stride and
-//                   alignment with rows of at least 16 bytes; K split over
-//                   workgroups where tiles are few.
-//   gemm_i8_tile64  64x64x64 tile, bounds-checked, for rows below 16 bytes.
+//                   alignment with K >= 16; K split over workgroups where
+//                   tiles are few.
+//   gemm_i8_tile64  64x64x64 tile, bounds-checked, for K < 16.
 // The requantize epilogue (round, shift, saturate, optional ReLU) is fused
 // into all of them.
 //
@@ -50,7 +50,7 @@ using miaie::launch;
 namespace flex = miaie::flex;
 
 // ------------------------------------------------------------ 64x64 tile
-// Bounds-checked fallback for rows of fewer than 16 bytes.
+// Bounds-checked fallback for K < 16 (and sizes of 2^30).
 template <bool B_NT>
 __global__ __launch_bounds__(256) void gemm_i8_tile64(const int8_t* __restrict__ A,
                                                       const int8_t* __restrict__ B,
@@ -137,8 +137,8 @@ __global__ __launch_bounds__(256) void gemm_i8_tile64(const int8_t* __restrict__
 }
 
 // Register-staged tiles (flex_tile.hpp): any size, stride and alignment with
-// rows of at least 16 bytes.  grid.x: output tiles, grid.y: the `splits`
-// workgroups that divide a tile's K; mode: shift, relu << 8, splits << 16 (one
+// K >= 16.  grid.x: output tiles, grid.y: the `splits` workgroups that divide a
+// tile's K; mode: shift, relu << 8, splits << 16 (one
 // argument: each costs the launch host time; what the loads need comes first,
 // in the 14 dwords that arrive in SGPRs).  Bound by the latency of the stages'
 // loads, and for few rows by reading B: 1000 x 2050 x 1000 NT (rows of 1000
@@ -146,7 +146,10 @@ __global__ __launch_bounds__(256) void gemm_i8_tile64(const int8_t* __restrict__
 // over 16 rows (4096 -> 11008 -> 4096, 90 MB of weights) 204.7 us in a
 // vectorised 64x64 kernel without a split and 29.2 (27.3 with K split 8
 // ways, 72 unsplit, on one box).
-template <class G, bool B_NT>
+//
+// ANY: 64-bit offsets, and a row-major B of any width (64x64 tiles alone):
+// 4096x10x4096 10.5 us, 44.0 in a vectorised 64x64 kernel without a split.
+template <class G, bool B_NT, bool ANY>
 __global__ __launch_bounds__(256, G::PER_CU) void gemm_i8_flex(const int8_t* __restrict__ A, const int8_t* __restrict__ B, int M,
                                                        int N, int K, int lda, int ldb, uint32_t mode,
                                                        int8_t* __restrict__ Y, int32_t* __restrict__ C, int ldy, int ldc,
@@ -168,12 +171,14 @@ __global__ __launch_bounds__(256, G::PER_CU) void gemm_i8_flex(const int8_t* __r
   for (int i = 0; i < G::NI; ++i)
 #pragma unroll
     for (int j = 0; j < G::NJ; ++j) acc[i][j] = v4i{0};
-  flex::RowsLoader<G, G::NA> la(A, m0, M, lda, K, tid);
+  using Off = std::conditional_t<ANY, size_t, uint32_t>;
+  flex::RowsLoader<G, G::NA, Off> la(A, m0, M, lda, K, tid);
   if constexpr (B_NT) {
-    flex::RowsLoader<G, G::NB> lb(B, n0, N, ldb, K, tid);
+    flex::RowsLoader<G, G::NB, Off> lb(B, n0, N, ldb, K, tid);
     flex::tile_loop<int8_t, G, false>(lds, la, lb, s0, s1, lane, wm, wn, acc);
   } else {
-    flex::ColsLoader<int8_t, G, false> lb(B, n0, N, ldb, K, tid);
+    std::conditional_t<ANY, flex::ColsLoaderAny<int8_t, G, false>, flex::ColsLoader<int8_t, G, false>> lb(B, n0, N, ldb,
+                                                                                                     K, tid);
     flex::tile_loop<int8_t, G, true>(lds, la, lb, s0, s1, lane, wm, wn, acc);
   }
   if (G::SPLITS && splits > 1 &&
@@ -421,10 +426,12 @@ static bool pipe_operands_ok(const int8_t* A, const int8_t* B, const int8_t* Y, 
          (!C || (aligned(C, 16) && ldc % 4 == 0));
 }
 
-// The register-staged kernel's conditions: rows of at least 16 bytes, and
-// 32-bit offsets within a tile.
-static bool flex_operands_ok(int N, int K, int lda, int ldb, int b_nt) {
-  return K >= 16 && (b_nt || N >= 16) && lda < (1 << 25) && ldb < (1 << 25);
+// The register-staged kernel's operands: rows of at least 16 bytes and 32-bit
+// offsets within a tile, or (Any) rows of A of 16 bytes alone.
+enum class FlexOperands { None, Any, Rows };
+static FlexOperands flex_operands(int N, int K, int lda, int ldb, int b_nt) {
+  if (K < 16 || K >= (1 << 30) || N >= (1 << 30)) return FlexOperands::None;
+  return (b_nt || N >= 16) && lda < (1 << 25) && ldb < (1 << 25) ? FlexOperands::Rows : FlexOperands::Any;
 }
 
 // How a product runs: pipelined tiles (pipe.bm > 0), register-staged ones
@@ -443,11 +450,15 @@ struct Route {
   PipePlan pipe;
   flex::Plan flex;
 };
-static Route route(miaie_ctx* ctx, int M, int N, int K, bool pipe_ok, bool flex_ok, bool can_split) {
+static Route route(miaie_ctx* ctx, int M, int N, int K, bool pipe_ok, FlexOperands ops, bool can_split) {
   Route r;
   if (pipe_ok) r.pipe = plan_pipe(M, N, K, ctx->cus);
+  if (ops == FlexOperands::Any) {
+    if (!r.pipe.bm) r.flex = flex::plan_any(M, N, K, ctx->cus, can_split, ctx->work_bytes);
+    return r;
+  }
   // (256-row tiles: enough of them that no split is better)
-  if (r.pipe.bm != 256 && flex_ok) {
+  if (r.pipe.bm != 256 && ops == FlexOperands::Rows) {
     r.flex = flex::plan(M, N, K, 1.0, ctx->cus, can_split, ctx->work_bytes);
     const double unit_us = (size_t)N * K > ((size_t)16 << 20) ? 0.7 : 0.5;
     if (r.pipe.bm && r.flex.bm && K <= (1 << 15) && r.flex.us < 0.75 * (1.5 + unit_us * r.pipe.cost))
@@ -459,7 +470,7 @@ static Route route(miaie_ctx* ctx, int M, int N, int K, bool pipe_ok, bool flex_
 }
 
 int plan_gemm_i8(miaie_ctx* ctx, int M, int N, int K, int dense_ok, miaie_gemm_plan* plan) {
-  const Route r = route(ctx, M, N, K, dense_ok, flex_operands_ok(N, K, K, N, false), true);
+  const Route r = route(ctx, M, N, K, dense_ok, flex_operands(N, K, K, N, false), true);
   const PipePlan& p = r.pipe;
   *plan = miaie_gemm_plan{};
   plan->threads = p.bm == 128 ? 512 : 256;
@@ -490,9 +501,10 @@ int plan_gemm_i8(miaie_ctx* ctx, int M, int N, int K, int dense_ok, miaie_gemm_p
 // Chooses the kernel.  Y and/or C may be NULL (not both).
 int launch_gemm_i8(miaie_ctx* ctx, const int8_t* A, const int8_t* B, int8_t* Y, int32_t* C, int M,
                    int N, int K, int lda, int ldb, int ldy, int ldc, int b_nt, int shift, int relu, bool keep_y) {
-  const bool pipe_ok = pipe_operands_ok(A, B, Y, C, K, lda, ldb, ldy, ldc), flex_ok = flex_operands_ok(N, K, lda, ldb, b_nt);
-  Route r = route(ctx, M, N, K, pipe_ok, flex_ok, true);
-  if (r.flex.splits > 1 && !may_split(ctx)) r = route(ctx, M, N, K, pipe_ok, flex_ok, false);
+  const bool pipe_ok = pipe_operands_ok(A, B, Y, C, K, lda, ldb, ldy, ldc);
+  const FlexOperands ops = flex_operands(N, K, lda, ldb, b_nt);
+  Route r = route(ctx, M, N, K, pipe_ok, ops, true);
+  if (r.flex.splits > 1 && !may_split(ctx)) r = route(ctx, M, N, K, pipe_ok, ops, false);
   const PipePlan& plan = r.pipe;
   const int dev = ctx->device;
   if (plan.bm && plan.nw) {
@@ -523,16 +535,28 @@ int launch_gemm_i8(miaie_ctx* ctx, const int8_t* A, const int8_t* B, int8_t* Y, 
   if (r.flex.bm) {
     const flex::Plan& f = r.flex;
     hipError_t e = hipSuccess;
-    flex::with_geom(f, [&](auto g) {
-      using G = typename decltype(g)::type;
-      const dim3 fg((unsigned)f.tiles, (unsigned)f.splits);
-      int8_t* const work = static_cast<int8_t*>(ctx->work);
-      const uint32_t mode = (uint32_t)(shift | relu << 8 | f.splits << 16);
-      e = b_nt ? launch<gemm_i8_flex<G, true>>(dev, fg, block, 0, ctx->stream, A, B, M, N, K, lda, ldb, mode, Y, C,
-                                               ldy, ldc, work)
-               : launch<gemm_i8_flex<G, false>>(dev, fg, block, 0, ctx->stream, A, B, M, N, K, lda, ldb, mode, Y, C,
-                                                ldy, ldc, work);
-    });
+    const dim3 fg((unsigned)f.tiles, (unsigned)f.splits);
+    int8_t* const work = static_cast<int8_t*>(ctx->work);
+    const uint32_t mode = (uint32_t)(shift | relu << 8 | f.splits << 16);
+    auto go = [&](auto k) {
+      e = launch<decltype(k)::value>(dev, fg, block, 0, ctx->stream, A, B, M, N, K, lda, ldb, mode, Y, C, ldy, ldc, work);
+    };
+    if (f.any)
+      flex::with_geom_any(f, [&](auto g) {
+        using G = typename decltype(g)::type;
+        if (b_nt)
+          go(kernel_t<gemm_i8_flex<G, true, true>>{});
+        else
+          go(kernel_t<gemm_i8_flex<G, false, true>>{});
+      });
+    else
+      flex::with_geom(f, [&](auto g) {
+        using G = typename decltype(g)::type;
+        if (b_nt)
+          go(kernel_t<gemm_i8_flex<G, true, false>>{});
+        else
+          go(kernel_t<gemm_i8_flex<G, false, false>>{});
+      });
     return check_launch(ctx, e, "gemm_i8_flex");
   }
   const hipError_t e =

@@ -133,6 +133,60 @@ def test_gemm_i8_flex_recorded(ctx):
         b.free()
 
 
+@pytest.mark.parametrize("N", [1, 2, 7, 10, 15])
+@pytest.mark.parametrize("M,K", [(1, 16), (1, 31), (70, 17), (64, 256), (300, 1000), (5, 4099)])
+@pytest.mark.parametrize("off", [0, 3])
+def test_gemm_i8_flex_narrow_b(ctx, M, N, K, off):
+    """B row-major with rows below one 16-byte load (a classifier's head),
+    operands exactly as long as the entry points say: dense, then with padded
+    rows at an odd address."""
+    print(f"[case] flex gemm {M}x{N}x{K} off {off} plan {ctx.plan_gemm_i8(M, N, K)}", flush=True)
+    rng = np.random.default_rng(M + 3 * N + 5 * K + off)
+    A, B = _i8(rng, M, K), _i8(rng, K, N)
+    Co = oracle.gemm_i8(A, B)
+    lda, ldb = K + off, N + off
+    bufA, bufB = _i8(rng, off + (M - 1) * lda + K), _i8(rng, off + (K - 1) * ldb + N)
+    for m in range(M):
+        bufA[off + m * lda: off + m * lda + K] = A[m]
+    for k in range(K):
+        bufB[off + k * ldb: off + k * ldb + N] = B[k]
+    dA, dB, dC, dY = ctx.upload(bufA), ctx.upload(bufB), ctx.empty((M, N), np.int32), ctx.empty((M, N), np.int8)
+    for rep in range(2):
+        ctx.copy_h2d(dC, np.full((M, N), 77, np.int32))
+        ctx.gemm_i8_i32(dA.ptr + off, dB.ptr + off, dC, M, N, K, lda, ldb, N)
+        if off == 0:
+            ctx.gemm_i8_rq(dA, dB, dY, M, N, K, 9, True)
+        ctx.wait(60_000)
+        assert np.array_equal(ctx.download(dC), Co), rep
+        assert off or np.array_equal(ctx.download(dY), oracle.requant(Co, 9, relu=True)), rep
+    for b in (dA, dB, dC, dY):
+        b.free()
+
+
+@pytest.mark.parametrize("layout", [mi.B_NN, mi.B_NT])
+@pytest.mark.parametrize("M,N,K,which", [(5, 33, 100, "A"), (5, 20, 19, "B"), (3, 3, 19, "B")])
+def test_gemm_i8_flex_long_rows(ctx, M, N, K, which, layout):
+    """A pitch of 2^25 bytes or more: offsets within a tile pass 32 bits'
+    range for larger tiles."""
+    rows_b, cols_b = (N, K) if layout == mi.B_NT else (K, N)
+    lda = (1 << 25) + 3 if which == "A" else K
+    ldb = (1 << 25) + 1 if which == "B" else cols_b
+    print(f"[case] flex gemm {M}x{N}x{K} lda {lda} ldb {ldb} layout {layout}", flush=True)
+    rng = np.random.default_rng(M + N + K + layout)
+    A, B = _i8(rng, M, K), _i8(rng, rows_b, cols_b)
+    dA, dB = ctx.empty(((M - 1) * lda + K,), np.int8), ctx.empty(((rows_b - 1) * ldb + cols_b,), np.int8)
+    for d, ld, mat in ((dA, lda, A), (dB, ldb, B)):
+        for r in range(mat.shape[0]):
+            row = np.ascontiguousarray(mat[r])
+            ctx._call("miaie_copy_h2d", d.ptr + r * ld, row.ctypes.data, mi._sz(row.nbytes))
+    dC = ctx.empty((M, N), np.int32)
+    ctx.gemm_i8_i32(dA, dB, dC, M, N, K, lda, ldb, N, layout)
+    ctx.wait(60_000)
+    assert np.array_equal(ctx.download(dC), oracle.gemm_i8(A, B, b_nt=layout == mi.B_NT))
+    for b in (dA, dB, dC):
+        b.free()
+
+
 # bf16 products are exact in fp32; each of the K additions is off by at most
 # 2^-24 / 2 of a partial sum, whose size stays below 6 times the results' rms
 # (partial sums of N(0, 1) terms scaled to it, over at most 6e6 results)
@@ -141,7 +195,11 @@ def _bf16_bar(K):
 
 
 BF16_SHAPES = [
-    (1, 8, 8),        # the smallest that runs here: one chunk of one row
+    (1, 8, 8),        # the smallest dense rows: one chunk of one row
+    (1, 1, 8),        # rows of B below one load, down to a column
+    (70, 3, 9),
+    (300, 7, 130),
+    (17, 5, 4100),    # ... split
     (1, 9, 9),        # a value past a chunk
     (16, 127, 127),   # skinny tile, one column short, a value short of a stage
     (17, 129, 128),
@@ -176,6 +234,28 @@ def test_gemm_bf16_flex(ctx, M, N, K):
         # the order of arrival of the splits does not matter
         assert first is None or np.array_equal(C, first), rep
         first = C
+    for b in (dA, dB, dC):
+        b.free()
+
+
+@pytest.mark.parametrize("M,N,K", [(2, 3, (1 << 24) + 8), (2, (1 << 24) + 5, 8)])
+def test_gemm_bf16_flex_long_rows(ctx, M, N, K):
+    """Rows of 2^24 values or more, few of them not 0 and whole numbers: the
+    sums are exact in any order."""
+    print(f"[case] flex bf16 {M}x{N}x{K}", flush=True)
+    rng = np.random.default_rng(1)
+    A, B = np.zeros((M, K), np.float32), np.zeros((K, N), np.float32)
+    ks = np.unique(np.concatenate([[0, K - 1], rng.integers(0, K, 500)]))
+    ns = np.unique(np.concatenate([[0, N - 1], rng.integers(0, N, 500)]))
+    A[:, ks] = rng.integers(-8, 9, (M, len(ks)))
+    B[np.ix_(ks, ns)] = rng.integers(-8, 9, (len(ks), len(ns)))
+    bits = lambda x: (x.view(np.uint32) >> 16).astype(np.uint16)  # exact: small whole numbers
+    dA, dB, dC = ctx.upload(bits(A)), ctx.upload(bits(B)), ctx.empty((M, N), np.float32)
+    ctx.gemm_bf16_f32(dA, dB, dC, M, N, K)
+    ctx.wait(60_000)
+    want = np.zeros((M, N), np.float32)
+    want[:, ns] = A[:, ks] @ B[np.ix_(ks, ns)]
+    assert np.array_equal(ctx.download(dC), want)
     for b in (dA, dB, dC):
         b.free()
 
