@@ -728,8 +728,8 @@ __global__ __launch_bounds__(256, G::PER_CU) void conv2d_i8_flex_walk(
   }
 }
 
-// Operands of fewer than 16 bytes, and above 2^31, and more tiles than a launch
-// takes: one thread per output element.
+// One thread per output element: a k of a few values (direct_us), operands of
+// fewer than 16 bytes or above 2^31, and more tiles than a launch takes.
 __global__ __launch_bounds__(256) void conv2d_i8_direct(const int8_t* __restrict__ X, const int8_t* __restrict__ W,
                                                         const uint8_t* __restrict__ shifts, int8_t* __restrict__ Y,
                                                         int N, int H, int Wd, int Cin, int Cout, int R, int S,
@@ -933,6 +933,20 @@ static flex::Plan flex_plan(miaie_ctx* ctx, long P, int Cin, int Cout, int R, in
   return f.splits > 1 && !may_split(ctx) ? flex::plan(P, Cout, k_bytes, 1.5, ctx->cus, false, 0) : f;
 }
 
+// Estimated time (us) of one thread per output: the chain of one output's loads,
+// or the outputs' loads and address arithmetic over all CUs (fitted to 296
+// layers of k <= 50 on 256 CUs; strided pixels cost more the deeper they are).
+// A k of a few values leaves a tile's stage and MFMAs mostly empty: against the
+// tile the register-staged kernel plans, 8x224x224x2 -> 1, 3x3: 7.6 and 13.2 us;
+// 8x112x112x4 -> 4, 1x1: 3.3 and 5.1; on the other side of the line
+// 8x224x224x3 -> 64, 7x7, stride 2: 919 and 11.3, 4x112x112x8 -> 8, 1x1: 4.6
+// and 5.2.
+static double direct_us(size_t outputs, int Cin, int R, int S, int cus) {
+  const double taps = (double)R * S, k = taps * Cin;
+  return 2.25 + std::max(0.1 * taps + 0.075 * k,
+                         (double)outputs * 256e-6 / cus * (2.0 + 0.23 * taps + (0.46 + 0.02 * Cin) * k));
+}
+
 static int launch_flex(miaie_ctx* ctx, const flex::Plan& f, const int8_t* X, const int8_t* W, const uint8_t* shifts,
                        int8_t* Y, int N, int H, int Wd, int Cin, int Cout, int R, int S, int stride, int pad, int Ho,
                        int Wo) {
@@ -1054,8 +1068,10 @@ int launch_conv2d_i8(miaie_ctx* ctx, const int8_t* X, const int8_t* W, const uin
                                                         Ho, Wo, 1);
     return check_launch(ctx, e, "conv2d_i8_igemm");
   }
-  if (f.bm) return launch_flex(ctx, f, X, W, shifts, Y, N, H, Wd, Cin, Cout, R, S, stride, pad, Ho, Wo);
-  // operands below 16 or above 2^31 bytes, or too many tiles
+  // (1.1: the plan's estimates of one stage are that much low)
+  const bool tiny_k = Cin <= 16 && R * S <= 50 && R * S * Cin <= 50;
+  if (f.bm && !(tiny_k && direct_us(P * Cout, Cin, R, S, ctx->cus) < 1.1 * f.us))
+    return launch_flex(ctx, f, X, W, shifts, Y, N, H, Wd, Cin, Cout, R, S, stride, pad, Ho, Wo);
   const size_t total = P * Cout;
   const size_t blocks = (total + 255) / 256;
   if (blocks >= ((size_t)1 << 31)) return fail(ctx, MIAIE_EINVAL, "conv2d: output too large for the direct kernel");

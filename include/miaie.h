@@ -163,7 +163,8 @@ MIAIE_API int miaie_plan_set_cus(miaie_ctx* ctx, int cus, int* previous);
  * Invalid shapes return MIAIE_EINVAL, as the entry point does. */
 #define MIAIE_CONV_ROWS 0   /* row-block kernel: 3x3, stride 1, Cin 32/64/128, Cout % 32 == 0 (rows in blocks of 64) */
 #define MIAIE_CONV_IGEMM 1  /* implicit-GEMM kernels: Cin % 32 == 0, Cout % 64 == 0 (large grids on register-staged tiles) */
-#define MIAIE_CONV_DIRECT 2 /* any shape: register-staged tiles (one thread per output for operands below 16 or above 2^31 bytes) */
+#define MIAIE_CONV_DIRECT 2 /* any shape: register-staged tiles (one thread per output for a k of a few values and operands
+                               below 16 or above 2^31 bytes) */
 #define MIAIE_CONV_TAPS 3   /* LDS-staged implicit GEMM over filter taps: Cin % 128 == 0, Cout % 64 == 0 */
 #define MIAIE_CONV_ROWS_DEEP 4 /* row-block kernel over 64-channel chunks of Cin: 3x3, stride 1, Cin % 64 == 0 up to 4096, Cout % 32 == 0 */
 MIAIE_API int miaie_plan_conv2d_i8(int N, int H, int W, int Cin, int Cout, int R, int S, int stride, int pad,

@@ -9,6 +9,7 @@ import pytest
 import aiehlc_amd as mi
 import oracle
 from aiehlc_amd import synth
+from hip_capture import Capture
 
 pytestmark = pytest.mark.gpu
 
@@ -302,7 +303,8 @@ def test_gemm_bf16_256_tiles_k_sweep(ctx, K):
 CONV_SHAPES = [
     # N, H, W, Cin, Cout, R, S, stride, pad
     (1, 4, 4, 1, 1, 1, 1, 1, 0),      # 16 bytes of X; W (1 byte) too small: one thread per output
-    (1, 4, 4, 1, 16, 1, 1, 1, 0),     # the smallest operands that run here
+    (1, 4, 4, 1, 16, 1, 1, 1, 0),     # 16 bytes of each, k of one value: one thread per output
+    (1, 4, 4, 1, 16, 5, 5, 1, 2),     # about the smallest that runs on tiles
     (2, 9, 11, 3, 64, 7, 7, 2, 3),    # a stem: runs of 21 bytes, pads on every side
     (1, 5, 5, 5, 3, 3, 3, 1, 1),      # pixels fewer than a tile, 3 channels
     (3, 7, 1, 16, 65, 3, 1, 1, 1),    # one column, R != S, one channel past a tile
@@ -381,3 +383,28 @@ def test_conv2d_i8_flex_of_2_30_pixels(ctx):
         assert np.array_equal(y, want[0, first - lo:first - lo + rows, :, 0]), first
     for b in (dX, dY, dW, dS):
         b.free()
+
+
+@pytest.mark.parametrize("shape,direct", [
+    ((8, 224, 224, 2, 1, 3, 3, 1, 1), True), ((4, 112, 112, 4, 4, 1, 1, 1, 0), True), ((1, 14, 14, 1, 20, 1, 1, 1, 0), True),
+    ((4, 112, 112, 16, 1, 1, 1, 1, 0), True), ((8, 112, 112, 1, 1, 5, 5, 1, 2), True), ((4, 112, 112, 8, 16, 1, 1, 1, 0), False),
+    ((8, 224, 224, 3, 16, 3, 3, 1, 1), False), ((4, 112, 112, 17, 1, 1, 1, 1, 0), False), ((1, 30, 30, 1, 2, 9, 9, 1, 4), False)])
+def test_conv2d_i8_of_a_tiny_k(shape, direct):
+    """A k of a few values: one thread per output where a tile's stage would be
+    mostly empty, at 256 CUs, tiles on the other side of the line."""
+    N, H, W, Cin, Cout, R, S, stride, pad = shape
+    print(f"[case] conv of a tiny k {shape}", flush=True)
+    rng = np.random.default_rng(sum(shape))
+    X, Wt = _i8(rng, N, H, W, Cin), _i8(rng, Cout, R, S, Cin)
+    sh = rng.integers(0, 13, size=Cout, dtype=np.uint8)
+    want = oracle.conv2d_nhwc_i8(X, Wt, sh, stride, pad)
+    cap = Capture()
+    c = cap.ctx
+    dX, dW, dS, dY = c.upload(X), c.upload(Wt), c.upload(sh), c.empty(want.shape, np.int8)
+    exe, grids = cap.record(lambda: c.conv2d_i8_nhwc(dX, dW, dS, dY, N, H, W, Cin, Cout, R, S, stride, pad))
+    assert (grids == [(-(-want.size // 256), 1, 1)]) == direct, grids
+    cap.replay(exe)
+    cap.sync()
+    assert np.array_equal(c.download(dY), want)
+    cap.ok(cap.hip.hipGraphExecDestroy(exe))
+    cap.close()
