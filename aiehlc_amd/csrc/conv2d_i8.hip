@@ -1040,13 +1040,21 @@ int launch_conv2d_i8(miaie_ctx* ctx, const int8_t* X, const int8_t* W, const uin
                                                                stride, pad, Ho, Wo, 1);
     return check_launch(ctx, e, "conv2d_i8_taps");
   }
-  // Three 64x64 tiles per CU or more: the register-staged kernel in place of
-  // the implicit GEMM on fragments from memory, which is the faster one below
-  // that (its workgroups start sooner), and the slower one above, where each
-  // fragment load touches 32 lines (4x112x112x96->256: 38.1 against 33.2 us;
-  // 8x64x64x160->512 1x1: 25.9 against 15.5; 2x56x56x64->64 stride 2, 25 tiles:
-  // 4.7 against 6.8).
-  const bool big = ((P + 63) / 64) * (size_t)((Cout + 63) / 64) >= 3 * (size_t)ctx->cus;
+  // From three 64x64 tiles per CU on, the register-staged kernel in place of the
+  // implicit GEMM on fragments from memory, whose fragment loads touch 32 lines
+  // each (4x112x112x96->256, 3x3: 38.1 against 33.2 us; 8x64x64x160->512, 1x1:
+  // 25.9 against 15.5).  (Below three its workgroups start sooner:
+  // 2x56x56x64->64, stride 2, 25 tiles: 4.7 against 6.8.)  But below six not for
+  // larger filters of stride 1, whose pixels come from the L1 and L2 for each
+  // further channel tile (32x28x28x96->128, 5x5, 3.1 tiles per CU: 26.1 against
+  // 32.9; with one channel tile, 1x250x250x224->64, 3x3: 27.1 against 23.8), nor
+  // over few channels (16x64x64x32->192, 7x7, stride 2: 15.6 against 19.6;
+  // 16x64x64x320->192, 3x3, stride 2: 33.2 against 26.7); and not at all over 32
+  // channels with half a 128x128 tile left over (8x112x112x32->192, 5x5: 50.7
+  // against 55.8).
+  const size_t tiles64 = ((P + 63) / 64) * (size_t)((Cout + 63) / 64), cus = (size_t)ctx->cus;
+  const bool early = R * S == 1 || (stride > 1 ? Cin >= 96 : Cin >= 128 && Cout == 64);
+  const bool big = tiles64 >= (early ? 3 : 6) * cus && !(R * S > 1 && stride == 1 && Cin == 32 && Cout % 128);
   flex::Plan f;
   if ((kernel != MIAIE_CONV_IGEMM || big) && flex_ok(N, H, Wd, Cin, Cout, R, S, pad, P))
     f = flex_plan(ctx, (long)P, Cin, Cout, R, S);

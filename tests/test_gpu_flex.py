@@ -408,3 +408,30 @@ def test_conv2d_i8_of_a_tiny_k(shape, direct):
     assert np.array_equal(c.download(dY), want)
     cap.ok(cap.hip.hipGraphExecDestroy(exe))
     cap.close()
+
+
+@pytest.mark.parametrize("shape,tiles", [
+    ((4, 28, 28, 96, 128, 5, 5, 1, 2), False), ((4, 28, 28, 96, 256, 5, 5, 1, 2), True), ((4, 56, 56, 96, 128, 3, 3, 2, 1), True),
+    ((4, 56, 56, 32, 128, 3, 3, 2, 1), False), ((8, 28, 28, 32, 192, 5, 5, 1, 2), False), ((4, 28, 28, 64, 128, 1, 1, 1, 0), True),
+    ((2, 28, 28, 64, 128, 1, 1, 1, 0), False)])
+def test_conv2d_i8_implicit_gemm_grids(ctx, shape, tiles):
+    """Layers of the implicit-GEMM shapes, planned for 32 CUs: three to six (and
+    nine) 64 x 64 tiles per CU on register-staged tiles (all in x) or on
+    fragments from memory (channel tiles in y)."""
+    N, H, W, Cin, Cout, R, S, stride, pad = shape
+    print(f"[case] implicit GEMM conv {shape}", flush=True)
+    rng = np.random.default_rng(sum(shape))
+    X, Wt = _i8(rng, N, H, W, Cin), _i8(rng, Cout, R, S, Cin)
+    sh = rng.integers(8, 13, size=Cout, dtype=np.uint8)
+    want = oracle.conv2d_nhwc_i8(X, Wt, sh, stride, pad)
+    cap = Capture()
+    c = cap.ctx
+    c.plan_set_cus(32)
+    dX, dW, dS, dY = c.upload(X), c.upload(Wt), c.upload(sh), c.empty(want.shape, np.int8)
+    exe, grids = cap.record(lambda: c.conv2d_i8_nhwc(dX, dW, dS, dY, N, H, W, Cin, Cout, R, S, stride, pad))
+    assert len(grids) == 1 and (grids[0][1] == 1) == tiles, grids
+    cap.replay(exe)
+    cap.sync()
+    assert np.array_equal(c.download(dY), want)
+    cap.ok(cap.hip.hipGraphExecDestroy(exe))
+    cap.close()
