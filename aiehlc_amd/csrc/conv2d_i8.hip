@@ -926,16 +926,27 @@ static bool flex_ok(int N, int H, int Wd, int Cin, int Cout, int R, int S, int p
          (R * cpr + 64) * cpr < ((size_t)1 << 32);
 }
 
-// its tile and split (bm = 0: more tiles than a launch takes)
+// its tile and split (bm = 0: more tiles than a launch takes).  64-byte stages
+// (half the time of a 256-byte one for a k of 48 bytes and up to 64 channels) are
+// left out where a walk over pixel tiles of longer stages is the faster one: over
+// more than four 64x64 tiles per CU, for a k of two of them (8x112x112x96->64, 1x1:
+// 8.3 and 7.3 us) and for whole 128-column tiles (16x64x64x64->128, 1x1: 8.8 and
+// 7.4).
 static flex::Plan flex_plan(miaie_ctx* ctx, long P, int Cin, int Cout, int R, int S) {
-  const long k_bytes = 16l * R * ((S * Cin + 15) / 16);
-  const flex::Plan f = flex::plan(P, Cout, k_bytes, 1.5, ctx->cus, true, ctx->work_bytes);
-  return f.splits > 1 && !may_split(ctx) ? flex::plan(P, Cout, k_bytes, 1.5, ctx->cus, false, 0) : f;
+  const long k_bytes = 16l * R * ((S * Cin + 15) / 16), tiles64 = ((P + 63) / 64) * ((Cout + 63) / 64);
+  const bool short_ok = tiles64 <= 4l * ctx->cus || (k_bytes <= flex::Short::KB && (Cout - 1) % 128 < 64);
+  auto plan = [&](bool can_split) {
+    return short_ok ? flex::plan(P, Cout, k_bytes, 1.5, ctx->cus, can_split, ctx->work_bytes)
+                    : flex::plan_of<flex::Skinny, flex::Small, flex::Large>(P, Cout, k_bytes, 1.5, ctx->cus, can_split,
+                                                                            ctx->work_bytes);
+  };
+  const flex::Plan f = plan(true);
+  return f.splits > 1 && !may_split(ctx) ? plan(false) : f;
 }
 
 // Estimated time (us) of one thread per output: the chain of one output's loads,
 // or the outputs' loads and address arithmetic over all CUs (fitted to 296
-// layers of k <= 50 on 256 CUs; strided pixels cost more the deeper they are).
+// layers of k <= 80 on 256 CUs; strided pixels cost more the deeper they are).
 // A k of a few values leaves a tile's stage and MFMAs mostly empty: against the
 // tile the register-staged kernel plans, 8x224x224x2 -> 1, 3x3: 7.6 and 13.2 us;
 // 8x112x112x4 -> 4, 1x1: 3.3 and 5.1; on the other side of the line
@@ -1076,9 +1087,11 @@ int launch_conv2d_i8(miaie_ctx* ctx, const int8_t* X, const int8_t* W, const uin
                                                         Ho, Wo, 1);
     return check_launch(ctx, e, "conv2d_i8_igemm");
   }
-  // (1.1: the plan's estimates of one stage are that much low)
-  const bool tiny_k = Cin <= 16 && R * S <= 50 && R * S * Cin <= 50;
-  if (f.bm && !(tiny_k && direct_us(P * Cout, Cin, R, S, ctx->cus) < 1.1 * f.us))
+  // (the plan's estimates of one stage are a tenth low, those of a walk over pixel
+  // tiles as much high or more)
+  const bool tiny_k = Cin <= 16 && R * S <= 80 && R * S * Cin <= 80;
+  const double actual = f.kb > flex::Short::KB && f.tiles > 4l * ctx->cus ? 0.9 : 1.1;
+  if (f.bm && !(tiny_k && direct_us(P * Cout, Cin, R, S, ctx->cus) < actual * f.us))
     return launch_flex(ctx, f, X, W, shifts, Y, N, H, Wd, Cin, Cout, R, S, stride, pad, Ho, Wo);
   const size_t total = P * Cout;
   const size_t blocks = (total + 255) / 256;
