@@ -441,11 +441,9 @@ static FlexOperands flex_operands(int N, int K, int lda, int ldb, int b_nt) {
 // from the last call, plus 1.5 us): a handful of 128x128 tiles over a long K,
 // which the register-staged kernel splits.  Pipelined against split:
 // 128x4096x11008 49.2 and 20.0 us, 256x4096x11008 48.8 and 35.0, 512x512x8192 NT
-// 29.4 and 12.6; on the other side of the line 256x4096x4096 19.2 and 16.3
-// first time, 12.0 and 16.1 repeated, 256x1024x2048 NT 7.3 either way.  Above
-// K = 2^15 the pipelined kernel stays, though a split would be faster there
-// too: the test of its rounding term at the largest K it takes (256x256x65472)
-// relies on its being planned.
+// 29.4 and 12.6, 256x256x65472 NT 295 and 26; on the other side of the line
+// 256x4096x4096 19.2 and 16.3 first time, 12.0 and 16.1 repeated, 256x1024x2048 NT
+// 7.3 either way.
 struct Route {
   PipePlan pipe;
   flex::Plan flex;
@@ -461,7 +459,7 @@ static Route route(miaie_ctx* ctx, int M, int N, int K, bool pipe_ok, FlexOperan
   if (r.pipe.bm != 256 && ops == FlexOperands::Rows) {
     r.flex = flex::plan(M, N, K, 1.0, ctx->cus, can_split, ctx->work_bytes);
     const double unit_us = (size_t)N * K > ((size_t)16 << 20) ? 0.7 : 0.5;
-    if (r.pipe.bm && r.flex.bm && K <= (1 << 15) && r.flex.us < 0.75 * (1.5 + unit_us * r.pipe.cost))
+    if (r.pipe.bm && r.flex.bm && r.flex.us < 0.75 * (1.5 + unit_us * r.pipe.cost))
       r.pipe = PipePlan{};
     else if (r.pipe.bm)
       r.flex = flex::Plan{};

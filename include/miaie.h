@@ -135,8 +135,8 @@ MIAIE_API int miaie_debug_unregister(miaie_ctx* ctx, const void* dev_ptr);
  * decomposition and tile choice that stand in for the reference's tiling
  * prototype, src/mlir/mlirfront/tilinglinalg/tilinglinalg.cpp:38-146).
  * miaie_gemm_i8_i32 runs the same plan, except that for K >= 2^16, where the
- * requantizing entry takes the register-staged kernel, it keeps the pipelined
- * one. */
+ * requantizing entry always takes the register-staged kernel, it may take a
+ * pipelined one. */
 typedef struct {
   int kernel;         /* MIAIE_KERNEL_* */
   int tile_m, tile_n; /* workgroup output tile */

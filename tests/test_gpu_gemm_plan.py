@@ -377,17 +377,29 @@ def test_random_shapes_match_the_oracle(ctx, M, N, K, layout, shift, relu, cus):
 # launcher holds to K < 2^16 (|acc| <= K * 2^14); K = 65472 is the largest
 # such K the pipelined kernels take, where an all -128 row times an all -128
 # column gives acc = 2^30 - 2^20 and, at s = 31, acc + 2^30 lies 2^20 below
-# 2^31.  K = 65536 takes the 64x64 kernel, whose requant rounds without the
+# 2^31.  K = 65536 takes register-staged tiles, whose requant rounds without the
 # add ((acc >> s) + bit s-1 of acc).  Rows 0-2 of A and columns 0-2 of B are
 # constant (-128, -128, 127) so that the top-left 3x3 block of accumulators
 # sits at the extremes +-K*2^14; the rest is random.
 @pytest.mark.parametrize("K,MN", [(65472, 256), (65536, 128)])
 @pytest.mark.parametrize("layout", [mi.B_NN, mi.B_NT])
-def test_requant_round_term_at_the_largest_k(ctx, K, MN, layout):
+@pytest.mark.parametrize("cus", [1, 0])
+def test_requant_round_term_at_the_largest_k(ctx, K, MN, layout, cus):
+    prev = ctx.plan_set_cus(cus) if cus else None
+    try:
+        _requant_round_term(ctx, K, MN, layout, cus)
+    finally:
+        if prev:
+            ctx.plan_set_cus(prev)
+
+
+def _requant_round_term(ctx, K, MN, layout, cus):
     M = N = MN
     plan = ctx.plan_gemm_i8(M, N, K)
     print(f"[case] requant boundary gemm {M}x{N}x{K} layout {layout} plan {plan}", flush=True)
-    assert (plan["kernel"] == mi.KERNEL_TILE64) == (K >= 1 << 16)
+    assert (plan["kernel"] == mi.KERNEL_TILE64) == (K >= 1 << 16 or not cus)
+    if not cus:
+        assert plan["workgroups"] > 16  # split: more than the 64 x 64 tiles of 256 x 256
     rng = np.random.default_rng(K + MN + layout)
     A = rng.integers(-128, 128, size=(M, K), dtype=np.int8)
     Bkn = rng.integers(-128, 128, size=(K, N), dtype=np.int8)
