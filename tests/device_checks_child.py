@@ -59,8 +59,11 @@ def main() -> int:
             b.free()
         cases.append(f"gemm_i8 {M}x{N}x{K} {'NT' if lay == mi.B_NT else 'NN'}")
 
-    for M, N, K in [(512, 256, 128), (256, 256, 96), (300, 264, 128), (100, 130, 40), (70, 70, 64)]:
-        say("gemm_bf16", M, N, K)
+    # (planned for one CU: the 256x256 kernels, for K of whole and odd k-tiles, and overlapping tiles)
+    for M, N, K, cus in [(512, 256, 128, 1), (256, 256, 96, 1), (300, 264, 128, 1), (512, 256, 128, 256), (100, 130, 40, 256),
+                         (70, 70, 64, 256), (70, 3, 130, 256), (300, 400, 2050, 256), (70, 513, 1163, 8), (5, 3, 7, 256)]:
+        say("gemm_bf16", M, N, K, "cus", cus)
+        ctx.plan_set_cus(cus)
         A = synth.bf16_normal((M, K), 1, 1.0 / np.sqrt(K))
         B = synth.bf16_normal((K, N), 2, 1.0 / np.sqrt(K))
         dA, dB, dC = ctx.upload(A), ctx.upload(B), ctx.empty((M, N), np.float32)
@@ -71,15 +74,55 @@ def main() -> int:
         assert err <= 1e-2, ("gemm_bf16", M, N, K, err)
         for b in (dA, dB, dC):
             b.free()
-        cases.append(f"gemm_bf16 {M}x{N}x{K}")
+        cases.append(f"gemm_bf16 {M}x{N}x{K} on {cus} CUs")
+    ctx.plan_set_cus(256)
+
+    # Register-staged tiles, operands unaligned and exactly as long as the
+    # entry point says: rows short and long, splits of each tile, B below one
+    # load.
+    for M, N, K, cus in [(65, 63, 33, 256), (70, 300, 2050, 256), (67, 111, 1414, 8), (70, 513, 2326, 8), (300, 300, 500, 1),
+                         (70, 7, 300, 256), (3, 1, 17, 256), (5, 9, 11, 256)]:
+        for lay in (mi.B_NN, mi.B_NT):
+            ctx.plan_set_cus(cus)
+            plan = ctx.plan_gemm_i8(M, N, K)
+            say("gemm_i8_i32 unaligned", M, N, K, lay, plan)
+            A, B = i8(M, K), (i8(N, K) if lay == mi.B_NT else i8(K, N))
+            off = 3
+            bufs = []
+            for mat in (A, B):
+                rows, cols = mat.shape
+                flat = i8(off + (rows - 1) * (cols + off) + cols)
+                for r in range(rows):
+                    flat[off + r * (cols + off): off + r * (cols + off) + cols] = mat[r]
+                bufs.append(ctx.upload(flat))
+            dA, dB = bufs
+            dC = ctx.empty((1 + M * N,), np.int32)
+            ctx.gemm_i8_i32(dA.ptr + off, dB.ptr + off, dC.ptr + 4, M, N, K, K + off, B.shape[1] + off, N, lay)
+            ctx.wait(120_000)
+            Co = oracle.gemm_i8(A, B, b_nt=lay == mi.B_NT)
+            assert np.array_equal(ctx.download(dC)[1:].reshape(M, N), Co), ("gemm_i8_i32", M, N, K, lay)
+            for b in (dA, dB, dC):
+                b.free()
+            cases.append(f"gemm_i8_i32 {M}x{N}x{K} {'NT' if lay == mi.B_NT else 'NN'} {plan['tile_m']}x{plan['tile_n']} "
+                         f"{plan['workgroups']} workgroups")
+    ctx.plan_set_cus(256)
 
     conv_shapes = [(1, 6, 56, 64, 64, 3, 3, 1, 1),     # row-block kernel
                    (1, 8, 8, 256, 64, 3, 3, 1, 1),      # chunked row-block kernel
                    (1, 16, 16, 256, 64, 3, 3, 2, 1),    # taps kernel, split K (workspace)
                    (1, 5, 9, 96, 64, 3, 3, 1, 1),       # implicit GEMM
-                   (1, 5, 5, 4, 8, 3, 3, 1, 1)]         # direct
-    for (N, H, W, Cin, Cout, R, S, st, pad) in conv_shapes:
-        say("conv", N, H, W, Cin, Cout, R, S, st, pad)
+                   (1, 5, 5, 4, 8, 3, 3, 1, 1),         # one thread per output: a k of a few values ...
+                   (1, 3, 2, 2, 3, 3, 3, 1, 1),         # ... and operands below 16 bytes
+                   (2, 9, 11, 3, 64, 7, 7, 2, 3),       # register-staged: runs of 21 bytes, padding on every side
+                   (1, 3, 3, 30, 40, 3, 3, 1, 4),       # ... padding wider than the filter
+                   (2, 20, 20, 130, 200, 3, 3, 1, 1),   # ... split K
+                   (1, 12, 12, 400, 520, 3, 3, 1, 1, 8),  # ... 128 x 128 tiles, split K (planned for 8 CUs)
+                   (1, 60, 62, 3, 20, 3, 3, 1, 1, 2),   # ... walked over, k of 48 bytes, a partial last tile (2 CUs)
+                   (1, 60, 62, 3, 20, 7, 7, 1, 3, 2),   # ... k of 224 bytes
+                   (1, 60, 62, 100, 128, 1, 1, 1, 0, 2)]  # ... 128 x 128 tiles
+    for (N, H, W, Cin, Cout, R, S, st, pad, *cus) in conv_shapes:
+        say("conv", N, H, W, Cin, Cout, R, S, st, pad, "cus", cus)
+        ctx.plan_set_cus(cus[0] if cus else 256)
         X, Wt = i8(N, H, W, Cin), i8(Cout, R, S, Cin)
         sh = rng.integers(8, 13, size=Cout, dtype=np.uint8)
         Ho, Wo = (H + 2 * pad - R) // st + 1, (W + 2 * pad - S) // st + 1
@@ -89,7 +132,8 @@ def main() -> int:
         assert np.array_equal(ctx.download(dY), oracle.conv2d_nhwc_i8(X, Wt, sh, st, pad)), ("conv", Cin, Cout)
         for b in (dX, dW, dS, dY):
             b.free()
-        cases.append(f"conv2d {mi.plan_conv2d_i8(N, H, W, Cin, Cout, R, S, st, pad)} {N}x{H}x{W}x{Cin}->{Cout}")
+        cases.append(f"conv2d {mi.plan_conv2d_i8(N, H, W, Cin, Cout, R, S, st, pad)} {N}x{H}x{W}x{Cin}->{Cout} {R}x{S}")
+    ctx.plan_set_cus(256)
 
     say("mlp")
     M, K, F, Nout = 256, 128, 512, 256

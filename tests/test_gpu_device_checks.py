@@ -31,7 +31,10 @@ def test_device_checked_build_passes_clean_runs_and_names_planted_faults():
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
     out = json.loads(r.stdout.strip().splitlines()[-1])
     print(json.dumps(out, indent=1), flush=True)
-    assert len(out["cases"]) >= 15
+    assert len(out["cases"]) >= 45
+    tiles = " ".join(out["cases"])  # every register-staged tile, the split ones among them
+    for tile in ("16x128", "64x64", "128x128"):
+        assert tile in tiles, tile
     kinds = " ".join(p["message"] for p in out["planted"])
     for word in ("copy", "store", "load"):
         assert word in kinds, kinds

@@ -75,6 +75,36 @@ def test_gemm_i8_flex_in_place_of_few_pipelined_tiles(ctx, M, N, K, layout):
     test_gemm_i8_flex(ctx, M, N, K, layout)
 
 
+# Splits of each tile (they differ in the size of a tile's slot and in how many
+# partial sums are in flight): M, N, K, CUs planned for (0: the device's), tile,
+# least splits.  bf16 has the same plan at half the K.
+SPLITS = [
+    (70, 300, 2050, 0, (16, 128), 2),
+    (67, 111, 1414, 8, (64, 64), 2),
+    (260, 1300, 2600, 0, (64, 64), 4),
+    (300, 400, 4100, 0, (64, 64), 6),
+    (70, 513, 2326, 8, (128, 128), 3),
+    (195, 4201, 3415, 0, (128, 128), 3),
+]
+
+
+def _planned_split(ctx, M, N, K, cus, tile, splits):
+    plan = ctx.plan_gemm_i8(M, N, K)
+    tiles = -(-M // tile[0]) * -(-N // tile[1])
+    assert (plan["tile_m"], plan["tile_n"]) == tile and plan["workgroups"] >= splits * tiles, plan
+
+
+@pytest.mark.parametrize("M,N,K,cus,tile,splits", SPLITS)
+@pytest.mark.parametrize("layout", [mi.B_NN, mi.B_NT])
+def test_gemm_i8_flex_splits_of_each_tile(ctx, M, N, K, cus, tile, splits, layout):
+    prev = ctx.plan_set_cus(cus or 256)
+    try:
+        _planned_split(ctx, M, N, K, cus, tile, splits)
+        test_gemm_i8_flex(ctx, M, N, K, layout)
+    finally:
+        ctx.plan_set_cus(prev)
+
+
 @pytest.mark.parametrize("M,N,K,layout", [(5, 40, 1000, mi.B_NN), (70, 90, 300, mi.B_NT), (130, 150, 48, mi.B_NN),
                                           (33, 100, 2100, mi.B_NT)])
 @pytest.mark.parametrize("off", [1, 3, 8])
@@ -239,6 +269,16 @@ def test_gemm_bf16_flex(ctx, M, N, K):
         b.free()
 
 
+@pytest.mark.parametrize("M,N,K,cus,tile,splits", [s for s in SPLITS if s[2] % 2 == 0])
+def test_gemm_bf16_flex_splits_of_each_tile(ctx, M, N, K, cus, tile, splits):
+    prev = ctx.plan_set_cus(cus or 256)
+    try:
+        _planned_split(ctx, M, N, K, cus, tile, splits)
+        test_gemm_bf16_flex(ctx, M, N, K // 2)
+    finally:
+        ctx.plan_set_cus(prev)
+
+
 @pytest.mark.parametrize("M,N,K", [(2, 3, (1 << 24) + 8), (2, (1 << 24) + 5, 8)])
 def test_gemm_bf16_flex_long_rows(ctx, M, N, K):
     """Rows of 2^24 values or more, few of them not 0 and whole numbers: the
@@ -314,6 +354,7 @@ CONV_SHAPES = [
     (1, 70, 130, 17, 66, 3, 3, 1, 1),  # rows longer than a pixel tile
     (40, 3, 2, 8, 24, 2, 2, 1, 0),    # many images within one pixel tile (two output columns, one row... 2 x 1)
     (1, 13, 13, 130, 70, 5, 5, 1, 2),  # k of 5 runs of 650 bytes: stages across runs, split
+    (2, 20, 20, 130, 200, 3, 3, 1, 1),  # 64 x 64 tiles, split
     (1, 3, 3, 7300, 5, 3, 3, 1, 1),   # k >= 2^16: the requant form without the rounding add
     (4, 64, 64, 3, 130, 3, 3, 1, 1),  # 256 x 2 tiles: 128 x 128
     (8, 96, 96, 32, 192, 1, 1, 1, 0),  # a large grid of the implicit-GEMM shapes
@@ -358,6 +399,16 @@ def test_conv2d_i8_flex(ctx, shape, off):
         assert (got[:off] == 77).all() and (got[-16:] == 77).all(), rep
     for b in (dX, dW, dS, dY):
         b.free()
+
+
+@pytest.mark.parametrize("off", [0, 5])
+def test_conv2d_i8_flex_128_split(ctx, off):
+    """128 x 128 tiles split over k, planned for 8 CUs."""
+    prev = ctx.plan_set_cus(8)
+    try:
+        test_conv2d_i8_flex(ctx, (1, 12, 12, 400, 520, 3, 3, 1, 1), off)
+    finally:
+        ctx.plan_set_cus(prev)
 
 
 def test_conv2d_i8_flex_of_2_30_pixels(ctx):
