@@ -1089,7 +1089,7 @@ int launch_conv2d_i8(miaie_ctx* ctx, const int8_t* X, const int8_t* W, const uin
   }
   // (the plan's estimates of one stage are a tenth low, those of a walk over pixel
   // tiles as much high or more)
-  const bool tiny_k = Cin <= 16 && R * S <= 80 && R * S * Cin <= 80;
+  const bool tiny_k = Cin <= 16 && R * S <= 80 && R * S * Cin <= 80 && P * Cout < ((size_t)1 << 32) - 256;  // (threads)
   const double actual = f.kb > flex::Short::KB && f.tiles > 4l * ctx->cus ? 0.9 : 1.1;
   if (f.bm && !(tiny_k && direct_us(P * Cout, Cin, R, S, ctx->cus) < actual * f.us))
     return launch_flex(ctx, f, X, W, shifts, Y, N, H, Wd, Cin, Cout, R, S, stride, pad, Ho, Wo);

@@ -411,27 +411,30 @@ def test_conv2d_i8_flex_128_split(ctx, off):
         ctx.plan_set_cus(prev)
 
 
-def test_conv2d_i8_flex_of_2_30_pixels(ctx):
-    """2^30 output pixels of one channel over two stages of k: 2^24 workgroups
-    with a 64 x 64 tile, one more than a launch takes.  Strips of rows at the
+@pytest.mark.parametrize("R,Cout", [(17, 1), (2, 5)])
+def test_conv2d_i8_flex_of_2_30_pixels(ctx, R, Cout):
+    """2^30 output pixels: of one channel over two stages of k, 2^24 workgroups
+    with a 64 x 64 tile, one more than a launch takes; of five channels and a k of
+    four values, more outputs than a launch has threads.  Strips of rows at the
     image's top, middle and end against the oracle."""
     H = W = 32768
-    R, pad, rows = 17, 8, 24
-    print(f"[case] flex conv {H}x{W}, {R}x{R}", flush=True)
+    pad, rows = R // 2, 24
+    print(f"[case] flex conv {H}x{W} -> {Cout}, {R}x{R}", flush=True)
     rng = np.random.default_rng(3)
-    Wt = _i8(rng, 1, R, R, 1)
-    dX, dY = ctx.empty((H, W), np.int8), ctx.empty((H, W), np.int8)
-    dW, dS = ctx.upload(Wt), ctx.upload(np.array([12], np.uint8))
+    Wt, sh = _i8(rng, Cout, R, R, 1), np.full(Cout, 12 if R > 2 else 7, np.uint8)
+    Ho = Wo = H + 2 * pad - R + 1
+    dX, dY = ctx.empty((H, W), np.int8), ctx.empty((Ho, Wo, Cout), np.int8)
+    dW, dS = ctx.upload(Wt), ctx.upload(sh)
     ctx.fill_i8(dX, H * W, 9)
-    ctx.conv2d_i8_nhwc(dX, dW, dS, dY, 1, H, W, 1, 1, R, R, 1, pad)
+    ctx.conv2d_i8_nhwc(dX, dW, dS, dY, 1, H, W, 1, Cout, R, R, 1, pad)
     ctx.wait(60_000)
-    for first in (0, 16380, H - rows):
+    for first in (0, 16380, Ho - rows):
         lo, hi = max(first - pad, 0), min(first + rows + pad, H)
-        x, y = np.empty((hi - lo, W), np.int8), np.empty((rows, W), np.int8)
+        x, y = np.empty((hi - lo, W), np.int8), np.empty((rows, Wo, Cout), np.int8)
         ctx._call("miaie_copy_d2h", x.ctypes.data, dX.ptr + lo * W, mi._sz(x.nbytes))
-        ctx._call("miaie_copy_d2h", y.ctypes.data, dY.ptr + first * W, mi._sz(y.nbytes))
-        want = oracle.conv2d_nhwc_i8(x.reshape(1, hi - lo, W, 1), Wt, np.array([12], np.uint8), 1, pad)
-        assert np.array_equal(y, want[0, first - lo:first - lo + rows, :, 0]), first
+        ctx._call("miaie_copy_d2h", y.ctypes.data, dY.ptr + first * Wo * Cout, mi._sz(y.nbytes))
+        want = oracle.conv2d_nhwc_i8(x.reshape(1, hi - lo, W, 1), Wt, sh, 1, pad)
+        assert np.array_equal(y, want[0, first - lo:first - lo + rows]), first
     for b in (dX, dY, dW, dS):
         b.free()
 
