@@ -152,7 +152,7 @@ class DeviceBuffer:
 
 
 def _addr(x) -> int | None:
-    # (a plain address first: the binding is a fifth of a small call's host time)
+    # (a plain address first: the usual operand of a small call)
     if type(x) is int or x is None:
         return x
     if isinstance(x, DeviceBuffer):
@@ -160,7 +160,7 @@ def _addr(x) -> int | None:
     return int(x)
 
 
-KERNEL_TILE64 = 0
+KERNEL_TILE64 = 0  # register-staged tiles (GemmPlan.tile_m x tile_n), or the 64x64 kernel for K < 16
 KERNEL_PIPE = 1
 KERNEL_PIPE_MIXED = 2  # 256x256 tiles, then 256x128 tiles over the last columns
 
@@ -227,8 +227,8 @@ class Context:
         self.device = device
         self._bufs: list[DeviceBuffer] = []
         # the compute entries' functions, looked up once: with the address
-        # check above, host time per call 3.03 -> 2.82 us (mm_window_i32), 3.55 ->
-        # 3.43 (int8 GEMM), 3.83 -> 3.55 (conv)
+        # check above, four calls of mm_window_i32 16.1 -> 14.9 us on one machine,
+        # 15.7 -> 15.5 on another (between processes they vary by as much)
         lib = self.lib
         self._f_window, self._f_i32, self._f_rq = lib.miaie_mm_window_i32, lib.miaie_gemm_i8_i32, lib.miaie_gemm_i8_rq
         self._f_bf16, self._f_conv, self._f_mlp = lib.miaie_gemm_bf16_f32, lib.miaie_conv2d_i8_nhwc, lib.miaie_mlp_i8

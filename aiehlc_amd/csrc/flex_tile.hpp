@@ -95,7 +95,9 @@ struct Plan {
 // has several.  Constants fitted to back-to-back launches on MI355X over 112
 // GEMM and conv shapes (10 to 4e10 multiply-adds; 12% rms error; the plan
 // picked is 1% slower than the best of all tiles and splits on average, 16% at
-// worst).  A tile of 32 x 128 was never more than 2% better than these three.
+// worst), operands in the caches: weights streamed from memory take up to a third
+// longer than estimated (16 x 11008 x 4096: 14.2 us, 11.2 estimated).  The
+// 64-byte stage's constants: 2700 products of a short k, 11% rms.  A tile of 32 x 128 was never more than 2% better than these three.
 // `cost`: stage cost relative to the int8 GEMM's (conv 1.5: its loads compute
 // their addresses).
 // (No divisions: this runs on the host for every call.)
@@ -464,8 +466,9 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t device_buffer(void* p, int byt
 // A tile whose stages are divided among `splits` workgroups: each writes its
 // accumulators to its slot of the context's workspace and counts itself in the
 // tile's counter; the last to arrive adds all of them in split order (so
-// floating-point sums do not depend on the order of arrival), sets the counter back to 0 for the next launch, and returns true:
-// it alone stores the tile.  No workgroup waits for another.  A second launch
+// floating-point sums do not depend on the order of arrival), sets the counter
+// back to 0 for the next launch, and returns true: it alone stores the tile.  No
+// workgroup waits for another.  A second launch
 // for the sum costs the device about 2 us; this costs the last workgroup one
 // round trip and its reads.
 template <class T, class G>

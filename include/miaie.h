@@ -123,7 +123,8 @@ MIAIE_API int miaie_debug_unregister(miaie_ctx* ctx, const void* dev_ptr);
 /* ---- GEMM planning ------------------------------------------------------ */
 
 #define MIAIE_KERNEL_TILE64 0     /* register-staged kernel, any shape and stride: tiles of 16x128, 64x64 or
-                                     128x128, K split over workgroups where tiles are few */
+                                     128x128, K split over workgroups where tiles are few (not while the
+                                     caller captures the stream); for K < 16 a bounds-checked 64x64 one */
 #define MIAIE_KERNEL_PIPE 1       /* pipelined tile_m x tile_n kernel, 4-stage LDS DMA pipeline; M >= tile_m,
                                      N >= tile_n, and N % 16 == 0 where tile_n does not divide N (the
                                      last tile row/column overlaps the one before it) */
