@@ -444,6 +444,10 @@ __global__ __launch_bounds__(256) void conv2d_i8_splitk_reduce(const int32_t* __
 // runs, each padded to whole 16-byte chunks (CPR per run).  The weights' chunks
 // are zero past their run, so what the pixels' hold there does not matter
 // (a neighbour's bytes); bytes outside the image row are zeroed.
+//
+// Workgroups per CU: the registers of eight (64 each) would spill.
+template <class G>
+constexpr int kPerCu = std::min(G::PER_CU, 6);
 struct RunShape {
   int H, Wd, Cin, R, Ho, Wo, stride, pad;
   int SC, CPR;                    // bytes per run (S * Cin), 16-byte chunks per run
@@ -585,7 +589,7 @@ struct WeightLoader {
 // requantize outweigh the MFMAs.  8x48x48x96 -> 146, 5x5 (10 stages): 29 us,
 // 19.9 ms with one thread per output.
 template <class G>
-__global__ __launch_bounds__(256, G::PER_CU) void conv2d_i8_flex(const int8_t* __restrict__ X, const int8_t* __restrict__ W,
+__global__ __launch_bounds__(256, kPerCu<G>) void conv2d_i8_flex(const int8_t* __restrict__ X, const int8_t* __restrict__ W,
                                                          const uint8_t* __restrict__ shifts, int8_t* __restrict__ Y,
                                                          RunShape k, int x_bytes, int P, int Cout,
                                                          int8_t* __restrict__ work, int splits) {
@@ -654,7 +658,7 @@ struct WalkGeom {
   static constexpr int LDS = G::A_BYTES + G::B_BYTES + G::BM * G::YP;
 };
 template <class G>
-__global__ __launch_bounds__(256, G::PER_CU) void conv2d_i8_flex_walk(
+__global__ __launch_bounds__(256, kPerCu<G>) void conv2d_i8_flex_walk(
     const int8_t* __restrict__ X, const int8_t* __restrict__ W, const uint8_t* __restrict__ shifts,
     int8_t* __restrict__ Y, RunShape k, int x_bytes, int P, int Cout, int step, int dn, int dh, int dw) {
   __shared__ __attribute__((aligned(1024))) int8_t lds[WalkGeom<G>::LDS];
@@ -972,10 +976,10 @@ static int launch_flex(miaie_ctx* ctx, const flex::Plan& f, const int8_t* X, con
     using G = typename decltype(g)::type;
     const long tn = (Cout + G::BN - 1) / G::BN, tm = f.tiles / tn;
     // one stage, and pixel tiles for more than one round of the workgroups
-    // that fit (by LDS and registers, 4 per CU, 2 of 128x128).  (Fewer
-    // workgroups, each with the same number of tiles: 12.7 us against 11.3 for
+    // that fit (kPerCu: 4 per CU of 64x64, 2 of 128x128, 6 with 64-byte stages).
+    // (Fewer workgroups, each with the same number of tiles: 12.7 us against 11.3 for
     // 8x224x224x3 -> 64, 7x7, stride 2.)
-    const long step = std::max(1l, (long)G::PER_CU * ctx->cus / tn);
+    const long step = std::max(1l, (long)kPerCu<G> * ctx->cus / tn);
     if (16 * R * k.CPR <= G::KB && tm > step) {
       const long pixels = step * G::BM;  // from one of a workgroup's tiles to its next
       e = launch<conv2d_i8_flex_walk<G>>(ctx->device, dim3((unsigned)(tn * step)), dim3(256), 0, ctx->stream, X, W,
