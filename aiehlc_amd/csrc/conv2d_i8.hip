@@ -437,6 +437,10 @@ __global__ __launch_bounds__(256) void conv2d_i8_splitk_reduce(const int32_t* __
 }
 
 // ------------------------------------------------------- register-staged kernel
+// Workgroups per CU: the registers of eight (64 each) would spill.
+template <class G>
+constexpr int kPerCu = std::min(G::PER_CU, 6);
+
 // Any shape, as an implicit GEMM on the register-staged tiles (flex_tile.hpp):
 // rows are output pixels, columns output channels.  For one filter row r the
 // S * Cin input bytes under the filter are one contiguous run of the image row
@@ -444,10 +448,6 @@ __global__ __launch_bounds__(256) void conv2d_i8_splitk_reduce(const int32_t* __
 // runs, each padded to whole 16-byte chunks (CPR per run).  The weights' chunks
 // are zero past their run, so what the pixels' hold there does not matter
 // (a neighbour's bytes); bytes outside the image row are zeroed.
-//
-// Workgroups per CU: the registers of eight (64 each) would spill.
-template <class G>
-constexpr int kPerCu = std::min(G::PER_CU, 6);
 struct RunShape {
   int H, Wd, Cin, R, Ho, Wo, stride, pad;
   int SC, CPR;                    // bytes per run (S * Cin), 16-byte chunks per run
@@ -932,13 +932,15 @@ static bool flex_ok(int N, int H, int Wd, int Cin, int Cout, int R, int S, int p
 
 // its tile and split (bm = 0: more tiles than a launch takes).  64-byte stages
 // (half the time of a 256-byte one for a k of 48 bytes and up to 64 channels) are
-// left out where a walk over pixel tiles of longer stages is the faster one: over
-// more than four 64x64 tiles per CU, for a k of two of them (8x112x112x96->64, 1x1:
-// 8.3 and 7.3 us) and for whole 128-column tiles (16x64x64x64->128, 1x1: 8.8 and
-// 7.4).
+// left out where a walk over pixel tiles of longer stages is the faster one: for a
+// k of two of them over more than four 64x64 tiles per CU (16x64x64x96->192, 1x1:
+// 11.9 and 10.0 us), and of one over whole 128-column tiles and more than 64 per
+// CU (8x224x224x64->256, 1x1: 47.9 and 43.6; at 24 per CU,
+// 8x112x112x64->256: 12.6 and 15.6).
 static flex::Plan flex_plan(miaie_ctx* ctx, long P, int Cin, int Cout, int R, int S) {
   const long k_bytes = 16l * R * ((S * Cin + 15) / 16), tiles64 = ((P + 63) / 64) * ((Cout + 63) / 64);
-  const bool short_ok = tiles64 <= 4l * ctx->cus || (k_bytes <= flex::Short::KB && (Cout - 1) % 128 < 64);
+  const bool short_ok = k_bytes <= flex::Short::KB ? (Cout - 1) % 128 < 64 || tiles64 <= 64l * ctx->cus
+                                                   : tiles64 <= 4l * ctx->cus;
   auto plan = [&](bool can_split) {
     return short_ok ? flex::plan(P, Cout, k_bytes, 1.5, ctx->cus, can_split, ctx->work_bytes)
                     : flex::plan_of<flex::Skinny, flex::Small, flex::Large>(P, Cout, k_bytes, 1.5, ctx->cus, can_split,

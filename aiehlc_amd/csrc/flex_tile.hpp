@@ -97,7 +97,8 @@ struct Plan {
 // picked is 1% slower than the best of all tiles and splits on average, 16% at
 // worst), operands in the caches: weights streamed from memory take up to a third
 // longer than estimated (16 x 11008 x 4096: 14.2 us, 11.2 estimated).  The
-// 64-byte stage's constants: 2700 products of a short k, 11% rms.  A tile of 32 x 128 was never more than 2% better than these three.
+// 64-byte stage's constants: 2700 products of a short k, 11% rms.  A tile of
+// 32 x 128 was never more than 2% better than these.
 // `cost`: stage cost relative to the int8 GEMM's (conv 1.5: its loads compute
 // their addresses).
 // (No divisions: this runs on the host for every call.)
